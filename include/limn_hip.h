@@ -171,10 +171,29 @@ int limn_hip_matmul_supported(int dtype, int64_t M, int64_t N, int64_t K, int64_
                               int64_t b_batch, int64_t b_k, int64_t b_n);
 
 /*
+ * limn_hip_matmul_add for float32, limn's default type: float32 operands, products, totals, result,
+ * bias and residual; one stride of each operand must be 1, the other any (no alignment past the
+ * element's). Replaces the same reference kernel as limn_hip_matmul (limn/cuda_emit.py:376-685).
+ * Same workspace rules, with limn_hip_contract_workspace(...) bytes.
+ */
+int limn_hip_contract(const void* a, const void* b, void* c, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
+                      int64_t a_batch, int64_t a_m, int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int64_t c_batch,
+                      int64_t c_m, int64_t c_n, int epilogue, const void* bias, int bias_dtype, int64_t bias_n,
+                      const void* residual, int64_t r_batch, int64_t r_m, int64_t r_n, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+int64_t limn_hip_contract_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K);
+
+/* 1 when limn_hip_contract takes this layout and is the faster way to compute it (a very small
+ * contraction is left to the general reduce kernels), else 0. */
+int limn_hip_contract_supported(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t a_batch, int64_t a_m,
+                                int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n);
+
+/*
  * A pre-bound launch list: the kernels of one recorded execution of a plan, replayed against new
  * buffers. Each step is one launch: a hipRTC module kernel (`function`, `grid` x `block`
  * threads, its arguments the kernel's parameters in order), a zero fill (pointer, bytes), or one
- * call of limn_hip_matmul (its 20 arguments before `stream`), limn_hip_matmul_add (27),
+ * call of limn_hip_matmul (its 20 arguments before `stream`), limn_hip_matmul_add or
+ * limn_hip_contract (27),
  * limn_hip_sdpa_fwd (13 before
  * `scale`), limn_hip_sdpa_bwd_q (15), limn_hip_sdpa_bwd_kv (16) or limn_hip_sdpa_bwd (17 before
  * `scale`, then passes, workspace and its size: 20), with `scale` in the step. An
@@ -192,6 +211,7 @@ enum {
   LIMN_HIP_STEP_SDPA_BWD_KV = 5,
   LIMN_HIP_STEP_MATMUL_ADD = 6,
   LIMN_HIP_STEP_SDPA_BWD = 7,
+  LIMN_HIP_STEP_CONTRACT = 8,
 };
 
 typedef struct {

@@ -225,7 +225,7 @@ int limn_hip_matmul_add(const void* a, const void* b, void* c, int dtype, int64_
   const int f32 = bias != nullptr && bias_dtype == LIMN_HIP_FLOAT32;
   if ((uintptr_t)bias % (f32 ? 4 : 2) != 0 || (uintptr_t)residual % 2 != 0)
     return fail(LIMN_HIP_EINVAL, "matmul_add: the bias and residual must be aligned to their element size");
-  MatmulAddends add = {bias, f32, bias_n, (const u16*)residual, r_batch, r_m, r_n, 0};
+  MatmulAddends add = {bias, f32, bias_n, residual, r_batch, r_m, r_n, 0};
   if (bias != nullptr && bias_n == 1 && (uintptr_t)bias % 16 == 0) add.vec |= 1;
   if (residual != nullptr && r_n == 1 && r_m % 8 == 0 && r_batch % 8 == 0 && (uintptr_t)residual % 16 == 0) add.vec |= 2;
   return launch_matmul(a, b, c, dtype, s, epilogue, add, workspace, workspace_bytes, (hipStream_t)stream);
@@ -246,6 +246,42 @@ int limn_hip_matmul_noalloc(const void* a, const void* b, void* c, int dtype, in
   void* ws = nullptr;
   if (need > 0 && (rc = scratch_address(&ws)) != LIMN_HIP_OK) return rc;
   return launch_matmul(a, b, c, dtype, s, epilogue, MatmulAddends{}, ws, need, (hipStream_t)stream);
+}
+
+int limn_hip_contract(const void* a, const void* b, void* c, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
+                      int64_t a_batch, int64_t a_m, int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int64_t c_batch,
+                      int64_t c_m, int64_t c_n, int epilogue, const void* bias, int bias_dtype, int64_t bias_n,
+                      const void* residual, int64_t r_batch, int64_t r_m, int64_t r_n, void* workspace,
+                      int64_t workspace_bytes, void* stream) {
+  MatmulShape s = {batch, M, N, K, a_batch, a_m, a_k, b_batch, b_k, b_n, c_batch, c_m, c_n};
+  if (dtype != LIMN_HIP_FLOAT32) return fail(LIMN_HIP_EUNSUPPORTED, "contract: takes float32, not dtype code %d", dtype);
+  if (batch < 1 || M < 1 || N < 1 || K < 1)
+    return fail(LIMN_HIP_EINVAL, "contract: sizes must be positive (batch %lld, M %lld, N %lld, K %lld)", (long long)batch,
+                (long long)M, (long long)N, (long long)K);
+  if (a == nullptr || b == nullptr || c == nullptr) return fail(LIMN_HIP_EINVAL, "contract: null buffer");
+  if (epilogue != MATMUL_EPILOGUE_NONE && epilogue != MATMUL_EPILOGUE_RELU)
+    return fail(LIMN_HIP_EINVAL, "contract: unknown epilogue %d", epilogue);
+  if (workspace_bytes < 0) return fail(LIMN_HIP_EINVAL, "contract: negative workspace size");
+  if (bias != nullptr && bias_dtype != dtype)
+    return fail(LIMN_HIP_EINVAL, "contract: the bias is of the output type, not dtype %d", bias_dtype);
+  if (!f32_layout_ok(s)) return fail(LIMN_HIP_EUNSUPPORTED, "contract: operands must be contiguous along m/n or k, within 2 GiB a batch entry");
+  if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)bias | (uintptr_t)residual) % 4 != 0)
+    return fail(LIMN_HIP_EINVAL, "contract: buffers must be aligned to their element size");
+  MatmulAddends add = {bias, 1, bias_n, residual, r_batch, r_m, r_n, 0};
+  return launch_matmul_f32(a, b, c, s, epilogue, add, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int64_t limn_hip_contract_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K) {
+  if (dtype != LIMN_HIP_FLOAT32 || batch < 1 || M < 1 || N < 1 || K < 1) return 0;
+  MatmulShape s = {batch, M, N, K, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  return f32_workspace_bytes(s);
+}
+
+int limn_hip_contract_supported(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t a_batch, int64_t a_m,
+                                int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n) {
+  if (dtype != LIMN_HIP_FLOAT32 || batch < 1 || M < 1 || N < 1 || K < 1) return 0;
+  MatmulShape s = {batch, M, N, K, a_batch, a_m, a_k, b_batch, b_k, b_n, 0, 0, 0};
+  return f32_layout_ok(s) && f32_pays(s);
 }
 
 int64_t limn_hip_matmul_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K) {

@@ -23,7 +23,7 @@ struct MatmulAddends {
   const void* bias;  // bias[n * bias_n], of the output type, or float32 rounded to it first
   int bias_f32;
   int64_t bias_n;
-  const u16* res;   // res[b * r_batch + m * r_m + n * r_n]
+  const void* res;  // res[b * r_batch + m * r_m + n * r_n], of the output type
   int64_t r_batch, r_m, r_n;
   int vec;          // bit 0: bias_n == 1 and 16-byte aligned; bit 1: res rows the same (r_n == 1)
 };
@@ -40,5 +40,13 @@ int64_t matmul_workspace_bytes(const MatmulShape& s);
 int matmul_layout_ok(const MatmulShape& s);
 int launch_matmul(const void* a, const void* b, void* c, int dtype, const MatmulShape& s, int epilogue,
                   const MatmulAddends& add, void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
+// float32 operands and result (matmul_f32.hip), any row stride and alignment.
+bool f32_layout_ok(const MatmulShape& s);
+bool f32_pays(const MatmulShape& s);  // faster than the general reduce kernels
+MatmulPlan plan_f32(const MatmulShape& s);
+int64_t f32_workspace_bytes(const MatmulShape& s);
+int launch_matmul_f32(const void* a, const void* b, void* c, MatmulShape s, int epilogue, const MatmulAddends& add,
+                      void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
 }  // namespace limn

@@ -63,7 +63,7 @@ template <typename T>
 __device__ __forceinline__ u16 add_terms(u16 t, const MatmulAddends& add, int64_t bz, int64_t row, int64_t col) {
   float x = T::unpack(t);
   if (add.bias != nullptr) x = x + T::unpack(bias_at<T>(add, col));
-  if (add.res != nullptr) x = T::unpack(add.res[bz * add.r_batch + row * add.r_m + col * add.r_n]) + x;
+  if (add.res != nullptr) x = T::unpack(((const u16*)add.res)[bz * add.r_batch + row * add.r_m + col * add.r_n]) + x;
   return T::pack(x);
 }
 
@@ -91,7 +91,7 @@ __device__ __forceinline__ u16x8 bias8(const MatmulAddends& add, int64_t col, in
 __device__ __forceinline__ u16x8 res8(const MatmulAddends& add, int64_t bz, int64_t row, int64_t col, int64_t N) {
   u16x8 v = zero8();
   if (add.res == nullptr) return v;
-  const u16* r = add.res + bz * add.r_batch + row * add.r_m;
+  const u16* r = (const u16*)add.res + bz * add.r_batch + row * add.r_m;
   if ((add.vec & 2) && col + 7 < N) return *(const u16x8*)(r + col);
 #pragma unroll
   for (int e = 0; e < 8; e++) v[e] = col + e < N ? r[(col + e) * add.r_n] : (u16)0;

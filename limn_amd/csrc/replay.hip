@@ -88,6 +88,16 @@ int run_step(const limn_hip_replay_step& s, int64_t i, const limn_hip_replay_arg
                                  (int)v[17], (const void*)(intptr_t)v[18], (int)v[19], v[20], (const void*)(intptr_t)v[21],
                                  v[22], v[23], v[24], (void*)(intptr_t)v[25], v[26], stream);
     }
+    case LIMN_HIP_STEP_CONTRACT: {
+      int rc = expect(s, i, 27, "contract");
+      if (rc != LIMN_HIP_OK) return rc;
+      int64_t v[27];
+      for (int k = 0; k < 27; k++) v[k] = bound(a[k], slots);
+      return limn_hip_contract((const void*)(intptr_t)v[0], (const void*)(intptr_t)v[1], (void*)(intptr_t)v[2], (int)v[3], v[4],
+                               v[5], v[6], v[7], v[8], v[9], v[10], v[11], v[12], v[13], v[14], v[15], v[16], (int)v[17],
+                               (const void*)(intptr_t)v[18], (int)v[19], v[20], (const void*)(intptr_t)v[21], v[22], v[23], v[24],
+                               (void*)(intptr_t)v[25], v[26], stream);
+    }
     case LIMN_HIP_STEP_SDPA_FWD: {
       int rc = expect(s, i, 13, "sdpa");
       if (rc != LIMN_HIP_OK) return rc;

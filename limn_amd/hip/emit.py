@@ -41,7 +41,7 @@ from dataclasses import dataclass, field, replace
 import numpy as np
 
 from limn_amd.hip import replay, runtime
-from limn_amd.seam import DType, Index, Instr, LoopNest, Node, Op, Opcode, Valid, accumulate_in, bfloat16, float16, float32, float64, int8, int16, int32
+from limn_amd.seam import DType, Index, Instr, LoopNest, Node, Op, Opcode, Valid, accumulate_in, bfloat16, float16, float32, float64, int8, int16, int32, realized
 
 THREADS = 256
 
@@ -437,7 +437,7 @@ def find_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
     if any(l.arg[2].bounds for l in loads):
         return None
     dtype = loads[0].value_type
-    if dtype not in (bfloat16, float16) or loads[1].value_type != dtype or shape.reduce_dtype != dtype:
+    if dtype not in (bfloat16, float16, float32) or loads[1].value_type != dtype or shape.reduce_dtype != dtype:
         return None
     if nest.kernel.target.dtype != dtype:
         return None
@@ -468,13 +468,21 @@ def find_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
     if batch > 1 and b_b == 0 and a_b == M * a_m and c_b == M * c_m:
         M, batch, a_b, c_b = M * batch, 1, 0, 0  # a shared right operand: one taller contraction
     con = Contraction(a_in, b_in, loads[0].arg[1].const, loads[1].arg[1].const, dtype, batch, M, N, K, a_b, a_m, a_k, b_b, b_k, b_n, c_b, c_m, c_n)
-    if con.a_offset % 8 or con.b_offset % 8:
-        return None
+    return con if contraction_supported(con) else None
+
+
+def contraction_supported(con: Contraction) -> bool:
+    """Whether liblimn_hip.so takes this contraction: the half widths with 16-byte aligned operand
+    rows (limn_hip_matmul), float32 with any (limn_hip_contract)."""
     from limn_amd.dtypes import ABI_CODE
 
-    lib = runtime.kernels()
-    ok = lib.limn_hip_matmul_supported(ABI_CODE[dtype], M, N, K, a_b, a_m, a_k, b_b, b_k, b_n)
-    return con if ok else None
+    lib, code = runtime.kernels(), ABI_CODE[con.dtype]
+    strides = (con.a_batch, con.a_m, con.a_k, con.b_batch, con.b_k, con.b_n)
+    if con.dtype is float32:
+        return bool(lib.limn_hip_contract_supported(code, con.batch, con.M, con.N, con.K, *strides))
+    if con.a_offset % 8 or con.b_offset % 8:
+        return False
+    return bool(lib.limn_hip_matmul_supported(code, con.M, con.N, con.K, *strides))
 
 
 def _vec_width(nest_shape: NestShape, bufs: Buffers, var: str, extent: int) -> int:
@@ -1353,7 +1361,51 @@ def plan_columns(nest: LoopNest, shape: NestShape, bufs: Buffers, cells: int, R:
                    notes={"columns": True, "parts": parts, "vec": vec})
 
 
-def plan_nest(nest: LoopNest, inlined: "InlineSet | None" = None, stream: bool = False) -> Planned:
+def deciding(nests: list[LoopNest]) -> set[Node]:
+    """The buffers of a plan whose values reach a comparison (CMPLT) that picks between other values,
+    through any nests and CUSTOM calls between. The mask of a relu's backward is such a comparison:
+    where a float32 sum is within its own rounding error of zero, another order of its additions
+    turns whole gradient elements on or off (one or two of the 8.4M hidden units of a 4096 x 512 ->
+    2048 layer moved its input's gradient by 8e-4 in 2-norm, against 1e-7 for the sums themselves).
+    Sums in this set keep the general reduce kernels' order of additions; the others (every gradient,
+    a last layer, logits, inference) are free to go to the matrix cores. A comparison that only picks
+    the larger or the smaller of the two values it compares (relu itself, maximum, minimum) has no
+    such jump and does not count."""
+    reached: set[Node] = set()
+    makers = {realized(n.kernel.target): n for n in nests}
+    work: list[Node] = []
+    for nest in nests:
+        taint: dict[str, frozenset[int]] = {}  # a value -> the inputs it depends on
+        # a CONST's name -> its value, so that two spellings of it match
+        same: dict[str, object] = {i.dest: ("const", i.arg[0]) for i in nest.instrs if i.opcode is Opcode.CONST}
+        compared: set[int] = set()
+        for i in nest.instrs:
+            if i.opcode is Opcode.LOAD:
+                taint[i.dest] = frozenset({int(i.arg[0][2:])})
+            elif i.opcode in (Opcode.ARITH, Opcode.CAST):
+                taint[i.dest] = frozenset().union(*(taint.get(s, frozenset()) for s in i.srcs))
+                if i.opcode is Opcode.ARITH and i.arg is Op.CMPLT:
+                    pair = {same.get(s, s) for s in i.srcs}
+                    users = [u for u in nest.instrs if i.dest in u.srcs]
+                    if not all(u.opcode is Opcode.ARITH and u.arg is Op.WHERE and u.srcs[0] == i.dest
+                               and i.dest not in u.srcs[1:] and {same.get(s, s) for s in u.srcs[1:]} == pair for u in users):
+                        compared |= taint[i.dest]
+        work += [nest.kernel.inputs[k] for k in sorted(compared)]
+    while work:
+        node = realized(work.pop())
+        if node in reached:
+            continue
+        reached.add(node)
+        if node in makers:
+            work += makers[node].kernel.inputs
+        elif node.op is Op.CUSTOM:
+            work += node.srcs
+    return reached
+
+
+def plan_nest(nest: LoopNest, inlined: "InlineSet | None" = None, stream: bool = False, ordered: bool = False) -> Planned:
+    """One nest's plan; `ordered` keeps a float32 sum of products on the general reduce kernels (see
+    `deciding`)."""
     """How one nest runs. With `inlined`, loads of the outputs of the producers it names are
     evaluated in place (see inline_producers); `stream` makes an elementwise nest's stores
     non-temporal (see streamed_outputs)."""
@@ -1368,7 +1420,7 @@ def plan_nest(nest: LoopNest, inlined: "InlineSet | None" = None, stream: bool =
     if shape.fold is None:
         return plan_elementwise(nest, shape, bufs, stream)
     con = find_contraction(nest, shape)
-    if con is not None:
+    if con is not None and not (ordered and con.dtype is float32):
         return Planned("", [], contraction=con, notes={"mfma": True})
     return plan_reduce(nest, shape, bufs)
 
@@ -1526,12 +1578,7 @@ def batch_sum_fold(reader: LoopNest, total: Node, con: Contraction) -> Contracti
     else:  # the reader's rows are the contraction's columns: c^T = b^T a^T, rows contiguous
         folded = Contraction(con.b_input, con.a_input, con.b_offset, con.a_offset, con.dtype, 1, con.N, con.M, K,
                              0, con.b_n, con.b_k, 0, con.a_k, con.a_m, 0, cols, rows)
-    from limn_amd.dtypes import ABI_CODE
-
-    lib = runtime.kernels()
-    ok = lib.limn_hip_matmul_supported(ABI_CODE[folded.dtype], folded.M, folded.N, folded.K, 0, folded.a_m, folded.a_k, 0,
-                                       folded.b_k, folded.b_n)
-    return folded if ok else None
+    return folded if contraction_supported(folded) else None
 
 
 def epilogue_pairs(nests: list[LoopNest], plans: list[Planned], kept: set | None) -> tuple[dict[int, int], dict[int, tuple], dict[int, Contraction]]:
@@ -2440,6 +2487,13 @@ def plan_program(nests: list[LoopNest], kept: set | None, custom_inputs: set | N
     Touches no GPU."""
     streamed = streamed_outputs(nests, kept, custom_inputs)
     plans = [plan_nest(n, stream=k in streamed) for k, n in enumerate(nests)]
+    ordered: set[int] = set()
+    if any(p.contraction is not None and p.contraction.dtype is float32 for p in plans):
+        compared = deciding(nests)
+        ordered = {k for k, n in enumerate(nests) if realized(n.kernel.target) in compared}
+        for k in ordered:
+            if plans[k].contraction is not None and plans[k].contraction.dtype is float32:
+                plans[k] = plan_nest(nests[k], ordered=True)
     pairs, addends, folds = epilogue_pairs(nests, plans, kept)
     fused = {j: i for i, j in pairs.items()}
     for j in fused:
@@ -2450,7 +2504,7 @@ def plan_program(nests: list[LoopNest], kept: set | None, custom_inputs: set | N
     inlined = InlineSet(nests, inline_producers(nests, plans, kept, pairs) | absorbed)
     for c, nest in enumerate(nests):
         if c not in inlined.producers and plans[c].launches and inlined.reached(nest):
-            plans[c] = plan_nest(nest, inlined, stream=c in streamed)
+            plans[c] = plan_nest(nest, inlined, stream=c in streamed, ordered=c in ordered)
     for j in inlined.producers:
         plans[j] = Planned("", [], notes={"inlined": True})
     chains = row_chains(nests, plans, custom_inputs, inlined, pairs) if rows else []
@@ -2608,14 +2662,18 @@ def _keep_runner(producer_inputs: dict, k: int):
 
 def _matmul_launcher(dev, con: Contraction, epilogue: int, adds: bool = False):
     """launch(inputs, out_ptr, bias_ptr, residual_ptr): the contraction through limn_hip_matmul, or
-    through limn_hip_matmul_add when `adds` (the residual read at the output's strides)."""
+    through limn_hip_matmul_add when `adds` (the residual read at the output's strides); a float32
+    one through limn_hip_contract either way."""
     from limn_amd.dtypes import ABI_CODE
 
     lib = dev.lib
     code = ABI_CODE[con.dtype]
     size = con.dtype.itemsize
     shape = (code, con.batch, con.M, con.N, con.K, con.a_batch, con.a_m, con.a_k, con.b_batch, con.b_k, con.b_n, con.c_batch, con.c_m, con.c_n, epilogue)
-    ws_bytes = int(lib.limn_hip_matmul_workspace(code, con.batch, con.M, con.N, con.K))
+    wide = con.dtype is float32
+    entry, step = (lib.limn_hip_contract, replay.STEP_CONTRACT) if wide else (lib.limn_hip_matmul_add, replay.STEP_MATMUL_ADD)
+    workspace = lib.limn_hip_contract_workspace if wide else lib.limn_hip_matmul_workspace
+    ws_bytes = int(workspace(code, con.batch, con.M, con.N, con.K))
     held: list = []  # the split-k workspace, allocated on first use and kept with the runner
 
     def launch(inputs: list, out: int, bias: int | None = None, res: int | None = None, bias_code: int = code) -> None:
@@ -2624,11 +2682,11 @@ def _matmul_launcher(dev, con: Contraction, epilogue: int, adds: bool = False):
         a = inputs[con.a_input].ptr + con.a_offset * size
         b = inputs[con.b_input].ptr + con.b_offset * size
         ws = held[0].ptr if held else None
-        if adds:
+        if adds or wide:
             args = (a, b, out, *shape, bias, bias_code, 1, res, con.c_batch, con.c_m, con.c_n, ws, ws_bytes)
-            runtime.check_limn(lib.limn_hip_matmul_add(*args, None))
+            runtime.check_limn(entry(*args, None))
             if dev.tape is not None:
-                dev.tape.append(replay.Launch(replay.STEP_MATMUL_ADD, args))
+                dev.tape.append(replay.Launch(step, args))
             return
         runtime.check_limn(lib.limn_hip_matmul(a, b, out, *shape, ws, ws_bytes, None))
         if dev.tape is not None:

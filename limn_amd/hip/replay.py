@@ -27,13 +27,14 @@ from dataclasses import dataclass, field
 import numpy as np
 
 (STEP_KERNEL, STEP_ZERO, STEP_MATMUL, STEP_SDPA_FWD, STEP_SDPA_BWD_Q, STEP_SDPA_BWD_KV, STEP_MATMUL_ADD,
- STEP_SDPA_BWD) = range(8)
+ STEP_SDPA_BWD, STEP_CONTRACT) = range(9)
 
 # which arguments of each step kind are device pointers (the rest are sizes, codes and flags)
 POINTER_ARGS = {
     STEP_ZERO: frozenset({0}),
     STEP_MATMUL: frozenset({0, 1, 2, 18}),
     STEP_MATMUL_ADD: frozenset({0, 1, 2, 18, 21, 25}),
+    STEP_CONTRACT: frozenset({0, 1, 2, 18, 21, 25}),
     STEP_SDPA_FWD: frozenset(range(6)),
     STEP_SDPA_BWD_Q: frozenset(range(8)),
     STEP_SDPA_BWD_KV: frozenset(range(9)),

@@ -1,0 +1,61 @@
+"""Which float32 sums of products a plan hands to the matrix cores (no GPU)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from limn_amd.seam import Op, Tensor, custom, float32, grad, lower_all, realized, schedule, topological
+from limn_amd.seam import device as limn_device
+
+emit = pytest.importorskip("limn_amd.hip.emit")
+
+rng = np.random.default_rng(5)
+
+
+@pytest.fixture(autouse=True)
+def on_numpy():
+    limn_device.set_device("numpy")
+    yield
+
+
+def lowered(sinks: list[Tensor]):
+    nodes = [t.node for t in sinks]
+    order = topological(nodes)
+    return lower_all(nodes, order, schedule(nodes, order)), {realized(s) for s in nodes}
+
+
+def float32_layer(train: bool, act) -> tuple[list, list]:
+    """A float32 Linear, `act`, Linear: the plan's roles for its sums, forward only or trained."""
+    x = Tensor(rng.standard_normal((512, 256)).astype(np.float32), requires_grad=True)
+    w1, w2 = (Tensor(rng.standard_normal(s).astype(np.float32), requires_grad=True) for s in ((256, 128), (128, 256)))
+    y = act(x @ w1) @ w2
+    sinks = [y, *grad((y * y).sum(), [x, w1, w2])] if train else [y]
+    nests, kept = lowered(sinks)
+    prog = emit.plan_program(nests, kept, set())
+    return nests, [p.contraction is not None for n, p in zip(nests, prog.plans) if n.kernel.ast.op is Op.SUM]
+
+
+def test_float32_sums_a_mask_reads_keep_their_order():
+    """A trained relu compares the first layer's sums to route gradients, so they stay on the general
+    reduce kernels; every other product goes to the matrix cores. Without a backward, or with an
+    activation that compares nothing, they all do."""
+    assert float32_layer(True, lambda h: h.relu())[1].count(False) == 1
+    assert all(float32_layer(False, lambda h: h.relu())[1])
+    assert all(float32_layer(False, lambda h: h.minimum(1.0))[1])
+    assert all(float32_layer(True, lambda h: h * h)[1])
+    assert not float32_layer(False, lambda h: (h > 0).where(h * 2.0, h))[1][0]
+
+
+def test_a_mask_reaches_back_through_attention():
+    """The sums behind a CUSTOM call whose result a mask reads keep their order too."""
+    q = Tensor(rng.standard_normal((4, 512, 64)).astype(np.float32))
+    w = Tensor(rng.standard_normal((64, 64)).astype(np.float32))
+    o, _ = custom("sdpa", ((q @ w).node, q.node, q.node), (True, 0.125), ((float32, (4, 512, 64)), (float32, (4, 512, 1))))
+    att = Tensor.from_node(o)
+    for picked, ordered in (((att > 0).where(att * 2.0, att), True), (att * 2.0, False)):
+        sinks = [picked.node]
+        order = topological(sinks)
+        nests = [n for n in lower_all(sinks, order, schedule(sinks, order))]
+        sums = [n for n in nests if n.kernel.ast.op is Op.SUM]
+        assert len(sums) == 1 and (realized(sums[0].kernel.target) in emit.deciding(nests)) is ordered
