@@ -424,6 +424,12 @@ def _flat_reduce(inner: list[tuple[str, int]], ta: dict[str, int], tb: dict[str,
 
 
 def find_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
+    """The dense contraction a reduce nest is, when liblimn_hip.so takes it."""
+    con = read_contraction(nest, shape)
+    return con if con is not None and contraction_supported(con) else None
+
+
+def read_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
     """The dense-contraction reading of a reduce nest (reference limn/cuda_emit.py:376-505
     detects the same shape, over one reduce var): a body of exactly two unmasked loads and their
     product, each load depending on every reduce var (flattened into one k, see _flat_reduce),
@@ -468,7 +474,7 @@ def find_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
     if batch > 1 and b_b == 0 and a_b == M * a_m and c_b == M * c_m:
         M, batch, a_b, c_b = M * batch, 1, 0, 0  # a shared right operand: one taller contraction
     con = Contraction(a_in, b_in, loads[0].arg[1].const, loads[1].arg[1].const, dtype, batch, M, N, K, a_b, a_m, a_k, b_b, b_k, b_n, c_b, c_m, c_n)
-    return con if contraction_supported(con) else None
+    return con
 
 
 def contraction_supported(con: Contraction) -> bool:
@@ -1139,6 +1145,89 @@ def plan_reduce(nest: LoopNest, shape: NestShape, bufs: Buffers) -> Planned:
     return Planned(source, launches, scratch_bytes=cells * parts * acc_dt.itemsize, notes={"parts": parts, "vec": vec})
 
 
+TILED_WAVES = 1024  # the fewest waves a register-tiled sum of products is launched with: one per SIMD
+
+
+def plan_tiled(nest: LoopNest, shape: NestShape, bufs: Buffers, con: "Contraction", general: Planned) -> Planned | None:
+    """A float32 sum of products c[m, n] = sum_k a[m, k] b[n, k] (both operands contiguous along k, as
+    x @ weight^T is) with exactly the additions of `general`, its plan in the lane-group form of
+    plan_reduce, and so its bits: lane u of G takes the VEC-wide chunks u, u + G, ... of k in order and
+    the G partial sums meet in a butterfly. Only what a group owns differs: a TILE x TILE block of
+    cells instead of one cell, so a row's chunk is loaded once for TILE cells. One cell a group is
+    bound by its loads (two a product); 8 x 8 cells leave a multiply and an add a product (the
+    rounding of each is part of the result, so no fused form) and a quarter of a load. The butterfly
+    exchanges halves of the block, each lane keeping the half its lane bit names, 63 exchanges for 64
+    cells; additions commute, so both halves hold what the full exchange would. The four waves of a
+    workgroup take neighbouring blocks, their rows shared through the L1.
+
+    Measured, one call, us, one cell a group -> blocks (rate): (4096 x 512 -> 2048) 7075 -> 258 (33
+    TFLOP/s, of 37 for a multiply and an add a product on every SIMD), 2048^3 14100 -> 459, 512^3 226 -> 13, (300 x 784 -> 300) 28 ->
+    12, (4096 x 32 -> 2048, a thread a cell) 151 -> 34. None where the plan has another form or the
+    blocks are too few to give every SIMD a wave (64 x 784 -> 128: 6.6 either way)."""
+    G, vec = general.notes.get("group", 0), general.notes.get("vec", 0)
+    if G == 1:  # a thread a cell, k in order: any chunk length keeps it
+        vec = 4 if con.K % 4 == 0 else 1
+    if not 1 <= G <= 64 or not vec or con.a_k != 1 or con.b_k != 1 or len(shape.inner) != 1 or shape.fold is not Op.ADD:
+        return None
+    if con.batch * con.M * con.N * con.K >= 1 << 62 or max(con.M * con.a_m, con.N * con.b_n) >= 1 << 31:
+        return None
+    for tile in (8, 4):
+        tm, tn = -(-con.M // tile), -(-con.N // tile)
+        if con.batch * tm * tn * G // 64 >= TILED_WAVES:
+            break
+    else:
+        return None
+    cells, chunks = tile * tile, con.K // vec
+    groups = THREADS // G  # blocks of cells per workgroup, as wm x wn
+    wm = 1 << ((groups.bit_length() - 1) // 2)
+    wn = groups // wm
+    grid_m, grid_n = -(-tm // wm), -(-tn // wn)
+    grid = con.batch * grid_m * grid_n
+    if grid > 1 << 20:
+        return None
+    lines = [signature(nest.name, nest, float32, bufs) + " {", "  const i64 bid_ = blockIdx.x, nblk_ = gridDim.x;"]
+    lines.append(f"  const int sub_ = threadIdx.x % {G}, own_ = threadIdx.x / {G};")
+    # workgroup b runs on XCD b % 8: contiguous runs of blocks per XCD
+    lines.append(f"  const int blk_ = (int)({f'bid_ % 8 * {grid // 8} + bid_ / 8' if grid % 8 == 0 else 'bid_'});")
+    lines.append(f"  const int n0 = (blk_ % {grid_n} * {wn} + own_ % {wn}) * {tile}, m0 = (blk_ / {grid_n} % {grid_m} * {wm} + own_ / {wn}) * {tile};")
+    lines.append(f"  const i64 bz = blk_ / {grid_n * grid_m};")
+    # rows past the edges read the last row; their cells are not stored
+    lines.append(f"  const float* pa[{tile}];")
+    lines.append(f"  const float* pb[{tile}];")
+    lines.append("#pragma unroll")
+    lines.append(f"  for (int i = 0; i < {tile}; i++) {{")
+    lines.append(f"    pa[i] = in{con.a_input} + {con.a_offset}LL + bz * {con.a_batch}LL + (i64)(m0 + i < {con.M} ? m0 + i : {con.M - 1}) * {con.a_m};")
+    lines.append(f"    pb[i] = in{con.b_input} + {con.b_offset}LL + bz * {con.b_batch}LL + (i64)(n0 + i < {con.N} ? n0 + i : {con.N - 1}) * {con.b_n};")
+    lines.append("  }")
+    lines.append(f"  float {', '.join(f'acc{v} = {literal(shape.identity, float32)}' for v in range(cells))};")
+    lines.append(f"  for (int c_ = sub_; c_ < {chunks}; c_ += {G}) {{")
+    lines.append(f"    float av[{tile}][{vec}], bv[{tile}][{vec}];")
+    lines.append("#pragma unroll")
+    lines.append(f"    for (int i = 0; i < {tile}; i++)")
+    lines.append("#pragma unroll")
+    lines.append(f"      for (int j = 0; j < {vec}; j++) {{ av[i][j] = pa[i][c_ * {vec} + j]; bv[i][j] = pb[i][c_ * {vec} + j]; }}")
+    for j in range(vec):
+        lines += [f"    acc{v} = fadd(acc{v}, av[{v // tile}][{j}] * bv[{v % tile}][{j}]);" for v in range(cells)]
+    lines.append("  }")
+    lines.append("  int at_ = 0;")
+    half, step = cells // 2, G // 2
+    while step:
+        if half:
+            lines.append(f"  const bool up{step} = sub_ & {step};")
+            for v in range(half):  # spelled out: as a loop, some compilers leave the array in scratch memory
+                lines.append(f"  acc{v} = fadd(up{step} ? acc{v + half} : acc{v}, (float)__shfl_xor(up{step} ? acc{v} : acc{v + half}, {step}));")
+            lines.append(f"  at_ += up{step} ? {half} : 0;")
+        else:
+            lines.append(f"  acc0 = fadd(acc0, (float)__shfl_xor(acc0, {step}));")
+        half, step = half // 2, step // 2
+    left = max(1, cells // G)
+    for v in range(left):
+        lines.append(f"  {{ const int m = m0 + (at_ + {v}) / {tile}, n = n0 + (at_ + {v}) % {tile};")
+        lines.append(f"    if (m < {con.M} && n < {con.N}) out[bz * {con.c_batch}LL + (i64)m * {con.c_m} + (i64)n * {con.c_n}] = acc{v}; }}")
+    lines.append("}")
+    return Planned("\n".join(lines), [Launch(nest.name, grid, THREADS, "io")], notes=mergeable(nest, bufs, lines, {"tiled": tile, "of": G}))
+
+
 def fold_parts(name: str, shape: NestShape, acc_t: str, out_dtype: DType, out_ref: str, wide: bool, cells: int, parts: int,
                ident: str, at: str) -> tuple[list[str], int]:
     """The kernel that folds each cell's partial totals (`scratch[at]`, `at` in g and p_) and
@@ -1419,10 +1508,13 @@ def plan_nest(nest: LoopNest, inlined: "InlineSet | None" = None, stream: bool =
     shape = read_nest(nest)
     if shape.fold is None:
         return plan_elementwise(nest, shape, bufs, stream)
-    con = find_contraction(nest, shape)
-    if con is not None and not (ordered and con.dtype is float32):
+    con = read_contraction(nest, shape)
+    if con is not None and not (ordered and con.dtype is float32) and contraction_supported(con):
         return Planned("", [], contraction=con, notes={"mfma": True})
-    return plan_reduce(nest, shape, bufs)
+    general = plan_reduce(nest, shape, bufs)
+    if con is not None and con.dtype is float32 and (inlined is None or not inlined.reached(nest)):
+        return plan_tiled(nest, read_nest(nest), bufs, con, general) or general
+    return general
 
 
 def _launcher(dev, fn: int, launch: Launch, nin: int):

@@ -121,3 +121,33 @@ def test_a_float32_linear_and_its_gradients_on_matrix_cores(hipdev, lead):
     want = [x2 @ w.T + b, dy2 @ w, dy2.T @ x2, dy2.sum(0)]
     for g, e in zip(got, want):
         np.testing.assert_allclose(g.reshape(e.shape), e, rtol=1e-5, atol=1e-5 * np.sqrt(np.mean(e * e)) * 4)
+
+
+# lane groups of 1, 8, 16, 32 and 64, chunks of 4, 2 and 1, ragged block edges, both block sizes, a batch, one operand twice
+@pytest.mark.parametrize("lead,k,n", [((4100,), 32, 1030), ((700,), 64, 700), ((333,), 130, 1290), ((512,), 512, 512), ((257,), 1021, 515),
+                                      ((300,), 784, 300), ((65,), 3000, 601), ((3, 130), 96, 530)], ids=str)
+def test_blocks_of_ordered_sums_give_the_bits_of_one_cell_a_group(hipdev, monkeypatch, lead, k, n):
+    """plan_tiled against the plan it replaces, forward sums that a comparison keeps off the matrix cores."""
+    from limn_amd.hip import emit
+
+    use_device(hipdev)
+    rng = np.random.default_rng(k)
+    x, w = Tensor(rng.standard_normal((*lead, k)).astype(np.float32)), Tensor(rng.standard_normal((n, k)).astype(np.float32))
+    kinds = []
+    blocks = emit.plan_tiled
+    monkeypatch.setattr(emit, "plan_tiled", lambda *a: kinds.append(blocks(*a)) or kinds[-1])
+
+    def run(b):
+        hipdev.plans.clear()
+        h = x @ b.transpose()
+        out = (h > 0).where(h * 2.0, h)
+        return [hipdev.copyout(buf) for buf in hipdev.execute([h.node, out.node])]
+
+    got = [run(w)] + ([run(x)] if len(lead) == 1 else [])
+    assert kinds[0] is not None and "tiled" in kinds[0].notes
+    monkeypatch.setattr(emit, "plan_tiled", lambda *a: None)
+    want = [run(w)] + ([run(x)] if len(lead) == 1 else [])
+    hipdev.plans.clear()
+    for g, e in zip(got, want):
+        for a, b in zip(g, e):
+            np.testing.assert_array_equal(a, b)
