@@ -44,4 +44,17 @@ int launch_mfma_bwd(const SdpaArgs& a, void* ws, int passes);  // LIMN_HIP_BWD_*
 bool rows_supports(int dtype, int64_t hd, int64_t hd_v);
 int launch_sdpa_rows(SdpaPass pass, const SdpaArgs& a);
 
+// The general-width calls whose float32 arithmetic runs on matrix cores (sdpa_wide.h): f32, f16 and
+// bf16, head dims in multiples of 4 up to 128, enough rows. launch_sdpa_rows hands them over.
+bool wide_takes(SdpaPass pass, const SdpaArgs& a);
+int launch_wide_f32(SdpaPass pass, const SdpaArgs& a);
+int launch_wide_f16(SdpaPass pass, const SdpaArgs& a);
+int launch_wide_bf16(SdpaPass pass, const SdpaArgs& a);
+// 32-row blocks from which a wave walks its streamed rows alone; fewer are split in four (split, 256
+// heads x 512 rows x 64 dims, 4096 blocks: 133 us forward, 173 alone; 8192 x 32 x 32: equal).
+constexpr int64_t WIDE_WAVES = 8192;
+// Workgroups of paired causal blocks from which blocks are paired (and 16 blocks a head); fewer leave
+// CUs idle and go a block each (8 heads x 256 rows: 12 us).
+constexpr int64_t WIDE_PAIRS = 512;
+
 }  // namespace limn

@@ -14,6 +14,10 @@
 // every tile, and the groups' partial results are combined at the end in a fixed butterfly
 // (the forward's as (max, total, accumulator) triples rescaled to the common max).
 //
+// Most f32, f16 and bf16 calls of this family go on to matrix cores (sdpa_wide.h, the same
+// arithmetic); these kernels keep float64, head dims that are no multiple of 4 or pass 128, and calls of
+// few rows (wide_takes).
+//
 // This family carries the widths the MFMA kernels do not (f32 and f64 above all, where the
 // reference's tolerances are 1e-5 and 1e-12): it computes in the dtype's compute width with
 // natural exp/log, folding streamed rows in ascending order.
@@ -410,7 +414,30 @@ bool rows_supports(int dtype, int64_t hd, int64_t hd_v) {
   return known && hd >= 1 && hd_v >= 1 && hd <= 256 && hd_v <= 256;
 }
 
+// Whether a call goes to the matrix-core kernels (sdpa_wide.h): what they can address, and enough
+// 32-row blocks that a wave each beats the lanes of the kernels above. One pass, us, rows / wide
+// (float32, causal; forward, dQ, dK/dV): 64 dims, 48 x 1024 rows at 32 dims 756/52, 912/66, 1140/98;
+// 8 heads x 128 rows of 64 13/9, 13/11, 13/13; 8 x 64 rows of 64 10.5/8.3, 10.7/9.8, 10.9/13.0;
+// 2 x 512 rows of 128 (32 blocks) 60/34, 66/48, 56/61; 32 x 64 rows of 128 27/16, 30/20, 31/28; 32 x 64
+// rows of 16 (64 blocks) 7.9/11.3, 5.1/5.9, 5.4/7.3, 128 x 64 of 16 10.0/9.3, 7.6/6.1, 8.5/7.5.
+bool wide_takes(SdpaPass pass, const SdpaArgs& a) {
+  if (a.dtype == LIMN_HIP_FLOAT64 || a.hd % 4 != 0 || a.hd_v % 4 != 0 || a.hd > 128 || a.hd_v > 128) return false;
+  if (a.t_q < 32 || a.t_k < 32) return false;  // a tile
+  const int64_t width = a.hd > a.hd_v ? a.hd : a.hd_v;
+  const int64_t blocks = a.batch * (((pass == SDPA_BWD_KV ? a.t_k : a.t_q) + 31) / 32);
+  if (blocks < (width <= 16 ? 128 : width <= 32 ? 1 : width <= 64 || pass != SDPA_BWD_KV ? 32 : 64)) return false;
+  // per-head byte offsets are 32-bit, below FAR and a tile past the end; loads are whole dwords
+  const int64_t rows = a.t_q > a.t_k ? a.t_q : a.t_k;
+  if ((rows + 256) * width * 4 >= (int64_t)0x70000000) return false;
+  const uintptr_t bits = (uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.dout;
+  return bits % 4 == 0;
+}
+
 int launch_sdpa_rows(SdpaPass pass, const SdpaArgs& a) {
+  if (wide_takes(pass, a))
+    return a.dtype == LIMN_HIP_FLOAT32   ? launch_wide_f32(pass, a)
+           : a.dtype == LIMN_HIP_FLOAT16 ? launch_wide_f16(pass, a)
+                                         : launch_wide_bf16(pass, a);
   switch (a.dtype) {
     case LIMN_HIP_FLOAT64:
       return launch_width<F64>(pass, a);

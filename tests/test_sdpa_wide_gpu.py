@@ -1,0 +1,150 @@
+"""Float32-arithmetic attention on matrix cores (csrc/sdpa_wide.h), through the C ABI on the GPU.
+
+Tolerance: every product, addition and exponential is float32 (half widths round once at the store);
+against float64 over a few thousand keys the parts of a sum are at most 2e-6 of its terms' size, the
+half widths' stores 2^-11 and 2^-8 of the value.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from limn_amd.hip import runtime
+
+pytestmark = pytest.mark.gpu
+
+CODE = {"float32": 1, "float16": 2, "bfloat16": 3}
+ROUND = {"float32": 0.0, "float16": 2.0**-10, "bfloat16": 2.0**-7}
+
+
+def stored(x, dtype):
+    from limn_amd.dtypes import from_storage, to_storage
+    from limn_amd import seam
+
+    t = getattr(seam, dtype)
+    bits = to_storage(np.ascontiguousarray(x, dtype=np.float32), t)
+    return bits, from_storage(bits.view(np.uint8), t, x.shape).astype(np.float64)
+
+
+def run(dev, dtype, q, k, v, do, mask, causal, scale):
+    """(out, lse, dq, dk, dv) of the device, as float64 values."""
+    from limn_amd.dtypes import from_storage
+    from limn_amd import seam
+
+    t = getattr(seam, dtype)
+    B, tq, hd = q.shape
+    tk, hv = v.shape[1:]
+    bufs = {}
+    for name, x in (("q", q), ("k", k), ("v", v), ("do", do), ("mask", mask)):
+        if x is not None:
+            bits = stored(x, dtype)[0]
+            bufs[name] = dev.alloc(bits.nbytes)
+            dev.copyin(bufs[name], bits)
+    size = t.itemsize
+    out, lse = dev.alloc(B * tq * hv * size), dev.alloc(B * tq * 4)
+    dq, dk, dv = dev.alloc(B * tq * hd * size), dev.alloc(B * tk * hd * size), dev.alloc(B * tk * hv * size)
+    m = bufs["mask"].ptr if mask is not None else None
+    sizes = (CODE[dtype], B, tq, tk, hd, hv, int(causal), scale, None)
+    runtime.check_limn(dev.lib.limn_hip_sdpa_fwd(bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, m, out.ptr, lse.ptr, *sizes))
+    o = from_storage(dev.copyout(out), t, (B, tq, hv)).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        delta = (stored(do, dtype)[1] * o).sum(-1).astype(np.float32)
+    d = dev.alloc(delta.nbytes)
+    dev.copyin(d, delta)
+    args = (bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, bufs["do"].ptr, lse.ptr, d.ptr, m)
+    runtime.check_limn(dev.lib.limn_hip_sdpa_bwd_q(*args, dq.ptr, *sizes))
+    runtime.check_limn(dev.lib.limn_hip_sdpa_bwd_kv(*args, dk.ptr, dv.ptr, *sizes))
+    dev.finish()
+    back = lambda b, shape: from_storage(dev.copyout(b), t, shape).astype(np.float64)
+    return o, dev.copyout(lse).view(np.float32).reshape(B, tq), back(dq, (B, tq, hd)), back(dk, (B, tk, hd)), back(dv, (B, tk, hv))
+
+
+def exact(dtype, q, k, v, do, mask, causal, scale):
+    q, k, v, do = (stored(x, dtype)[1] for x in (q, k, v, do))
+    s = q @ k.swapaxes(1, 2) * scale
+    if causal:
+        s = np.where(np.tril(np.ones(s.shape[1:], bool)), s, -np.inf)
+    if mask is not None:
+        s = np.where(mask[:, None, :] != 0, s, -np.inf)
+    top = s.max(-1, keepdims=True)
+    p = np.exp(s - top)
+    total = p.sum(-1, keepdims=True)
+    p /= total
+    o = p @ v
+    dp = do @ v.swapaxes(1, 2)
+    ds = p * (dp - (do * o).sum(-1, keepdims=True)) * scale
+    return o, (top + np.log(total))[..., 0], ds @ k, ds.swapaxes(1, 2) @ q, p.swapaxes(1, 2) @ do
+
+
+# (batch, t_q, t_k, hd, hd_v, causal, masked): block and tile edges (32), one to many tiles a wave, padded
+# dims at each width (32, 64, 96, 128), unequal dims, paired causal blocks (512 units), a wave a block (8192 blocks)
+CASES = [
+    (33, 32, 32, 32, 32, True, False), (5, 65, 65, 20, 28, True, True), (40, 33, 200, 64, 64, False, True), (9, 300, 129, 80, 64, False, False),
+    (70, 127, 127, 128, 128, True, False), (6, 400, 400, 96, 96, True, True), (130, 50, 34, 16, 4, False, False), (64, 513, 513, 32, 32, True, False),
+    (4100, 64, 64, 32, 32, True, False), (8200, 32, 40, 4, 8, False, True),
+]
+
+
+@pytest.mark.parametrize("dtype", list(CODE))
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_matches_float64(hipdev, case, dtype):
+    B, tq, tk, hd, hv, causal, masked = case
+    rng = np.random.default_rng(tq + hd)
+    q, k, v, do = (rng.standard_normal(s) for s in ((B, tq, hd), (B, tk, hd), (B, tk, hv), (B, tq, hv)))
+    mask = (rng.random((B, tk)) < 0.7).astype(np.float64) if masked else None
+    if masked:
+        mask[:, 0] = 1
+    narrow = dtype != "float32" and hd == hv and hd in (64, 128)  # the 16-bit family's backward
+    for scale in (hd**-0.5,) if narrow else (hd**-0.5, -0.3):
+        got, want = run(hipdev, dtype, q, k, v, do, mask, causal, scale), exact(dtype, q, k, v, do, mask, causal, scale)
+        for name, g, w in zip(("out", "lse", "dq", "dk", "dv"), got, want):
+            # delta is summed from the rounded output: its rounding reaches dq and dk at the size of the row
+            rel = 1e-5 + (ROUND[dtype] if name != "lse" else 0.0)
+            np.testing.assert_allclose(g, w, rtol=rel, atol=rel * max(1.0, np.abs(w).max()), err_msg=name)
+
+
+def test_hidden_keys_keep_their_garbage_to_themselves(hipdev):
+    """Masked keys may hold NaN or infinities: no live row or key sees them."""
+    B, t, d = 8, 150, 64
+    rng = np.random.default_rng(0)
+    q, k, v, do = (rng.standard_normal((B, t, d)) for _ in range(4))
+    mask = np.ones((B, t))
+    mask[:, 100:] = 0
+    clean = run(hipdev, "float32", q, k, v, do, mask, False, 0.125)
+    k[:, 100:], v[:, 100:] = np.nan, np.inf
+    got = run(hipdev, "float32", q, k, v, do, mask, False, 0.125)
+    for g, c in zip(got[:3], clean[:3]):
+        np.testing.assert_array_equal(g, c)
+    for g, c in zip(got[3:], clean[3:]):
+        np.testing.assert_array_equal(g[:, :100], c[:, :100])
+
+
+@pytest.mark.parametrize("at", [3, 40, 95])
+def test_a_causal_row_sees_no_later_infinity(hipdev, at):
+    """An infinity in one value row and a NaN in one dO row: rows before (queries) and keys after (for dO)
+    stay as they were, and the rows that do read it are not finite."""
+    B, t, d = 12, 96, 32
+    rng = np.random.default_rng(1)
+    q, k, v, do = (rng.standard_normal((B, t, d)) for _ in range(4))
+    clean = run(hipdev, "float32", q, k, v, do, None, True, 0.2)
+    broken = v.copy()
+    broken[:, at, 5] = np.inf
+    got = run(hipdev, "float32", q, k, broken, do, None, True, 0.2)
+    np.testing.assert_array_equal(got[0][:, :at], clean[0][:, :at])
+    assert np.isposinf(got[0][:, at:, 5]).all()
+    np.testing.assert_array_equal(np.delete(got[0], 5, axis=2), np.delete(clean[0], 5, axis=2))
+    np.testing.assert_array_equal(got[2][:, :at], clean[2][:, :at])  # dq of the rows before it
+    broken = do.copy()
+    broken[:, at, 7] = np.nan
+    got = run(hipdev, "float32", q, k, v, broken, None, True, 0.2)
+    np.testing.assert_array_equal(got[4][:, at + 1 :], clean[4][:, at + 1 :])  # dv of keys its query does not see
+    assert np.isnan(got[4][:, : at + 1, 7]).all()
+
+
+def test_same_bits_twice(hipdev):
+    rng = np.random.default_rng(2)
+    x = [rng.standard_normal((64, 520, 32)) for _ in range(4)]
+    a, b = (run(hipdev, "float32", *x, None, True, 0.2) for _ in range(2))
+    for p, q in zip(a, b):
+        np.testing.assert_array_equal(p, q)
