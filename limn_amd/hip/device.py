@@ -36,15 +36,23 @@ SDPA, SDPA_BWD_Q, SDPA_BWD_KV = "sdpa", "sdpa_bwd_q", "sdpa_bwd_kv"
 BWD_BOTH = 3  # LIMN_HIP_BWD_BOTH: limn_hip_sdpa_bwd runs both passes
 
 
-# One workgroup per table entry (value, target, bytes <= 64 KiB, 16-byte aligned starts): 16-byte
-# copies, then the entry's tail byte by byte.
+# One table row per commit (value, target, bytes, the commit's first workgroup); a workgroup copies
+# 64 KiB of its commit (16-byte aligned starts): 16-byte copies, then a tail byte by byte. It finds
+# its row by bisection over the first workgroups, uniform scalar loads, so the host lists the
+# commits and not their chunks: an optimizer step over 12.6 M parameters and their moments (30
+# commits, 2324 chunks) spent 0.45 ms of host time on a row per chunk.
 COMMIT_SOURCE = r"""
-extern "C" __global__ void limn_commit_batch(const long long* __restrict__ table, long long entries) {
-  const long long e = blockIdx.x;
-  if (e >= entries) return;
-  const char* src = (const char*)table[3 * e];
-  char* dst = (char*)table[3 * e + 1];
-  const long long n = table[3 * e + 2], whole = n / 16;
+extern "C" __global__ void limn_commit_batch(const long long* __restrict__ table, long long commits) {
+  long long lo = 0, hi = commits;  // the last row whose first workgroup is at or before this one
+  while (hi - lo > 1) {
+    const long long mid = (lo + hi) / 2;
+    if (table[4 * mid + 3] <= (long long)blockIdx.x) lo = mid; else hi = mid;
+  }
+  const long long off = ((long long)blockIdx.x - table[4 * lo + 3]) << 16, left = table[4 * lo + 2] - off;
+  if (left <= 0) return;
+  const char* src = (const char*)table[4 * lo] + off;
+  char* dst = (char*)table[4 * lo + 1] + off;
+  const long long n = left < (1 << 16) ? left : 1 << 16, whole = n / 16;
   for (long long i = threadIdx.x; i < whole; i += blockDim.x) ((uint4*)dst)[i] = ((const uint4*)src)[i];
   for (long long i = whole * 16 + threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
 }
@@ -128,7 +136,8 @@ class HipDevice(CompiledDevice):
         self._commits: list[tuple[Buffer, Buffer]] = []
         self._commit_targets: set[int] = set()
         self._committed: list[tuple[Buffer, Buffer]] = []  # launched, kept alive until the barrier
-        self._commit_table: tuple[int, int, Buffer] | None = None  # (pinned host ptr, entries, device copy)
+        self._commit_table: tuple[int, int, Buffer] | None = None  # (pinned host ptr, rows, device copy)
+        self._commit_kernel: int | None = None
         self.custom[SDPA] = self._sdpa_runner
         self.custom[SDPA_BWD_Q] = self._sdpa_runner
         self.custom[SDPA_BWD_KV] = self._sdpa_runner
@@ -323,26 +332,26 @@ class HipDevice(CompiledDevice):
     COMMIT_CHUNK = 1 << 16  # bytes per workgroup of the commit kernel
 
     def _flush_commits(self) -> None:
-        """Launch the queued commits as one kernel over a (value, target, bytes) table. The queue is
+        """Launch the queued commits as one kernel over a table of them (COMMIT_SOURCE). The queue is
         taken first, so an allocation failure below (whose trim() finishes the batch) finds
         nothing left to flush; a grown table is allocated before the old one is released."""
         if not self._commits:
             return
         commits, self._commits, self._commit_targets = self._commits, [], set()
-        entries = []
-        for target, value in commits:
-            for off in range(0, value.nbytes, self.COMMIT_CHUNK):
-                entries.append((value.ptr + off, target.ptr + off, min(self.COMMIT_CHUNK, value.nbytes - off)))
+        table = np.empty((len(commits), 4), dtype=np.int64)
+        blocks = 0
+        for row, (target, value) in zip(table, commits):
+            row[:] = value.ptr, target.ptr, value.nbytes, blocks
+            blocks += -(-value.nbytes // self.COMMIT_CHUNK)
         if self._committed:
             # the pinned table of an earlier launch in this batch may not have been read yet
             check(self.api.hipStreamSynchronize(None), "waiting for a commit table")
-        table = np.array(entries, dtype=np.int64)
         host, cap, dev_table = self._commit_table or (0, 0, None)
-        if cap < len(entries):
-            cap = max(len(entries), 2 * cap, 1024)
-            grown = self._alloc(cap * 24)
+        if cap < len(commits):
+            cap = max(len(commits), 2 * cap, 1024)
+            grown = self._alloc(cap * 32)
             ptr = ctypes.c_void_p()
-            check(self.api.hipHostMalloc(ctypes.byref(ptr), cap * 24, 0), "allocating a pinned commit table")
+            check(self.api.hipHostMalloc(ctypes.byref(ptr), cap * 32, 0), "allocating a pinned commit table")
             if host:
                 check(self.api.hipStreamSynchronize(None), "waiting for a commit table")
                 self.api.hipHostFree(ctypes.c_void_p(host))
@@ -350,10 +359,11 @@ class HipDevice(CompiledDevice):
             self._commit_table = (host, cap, dev_table)
         ctypes.memmove(host, table.ctypes.data, table.nbytes)
         check(self.api.hipMemcpyAsync(ctypes.c_void_p(dev_table.ptr), ctypes.c_void_p(host), table.nbytes, HOST_TO_DEVICE, None), "uploading a commit table")
-        fn = runtime.load_functions(COMMIT_SOURCE, ["limn_commit_batch"])["limn_commit_batch"]
-        args = (ctypes.c_void_p * 2)(ctypes.c_void_p(dev_table.ptr), ctypes.c_void_p(len(entries)))
+        if self._commit_kernel is None:
+            self._commit_kernel = runtime.load_functions(COMMIT_SOURCE, ["limn_commit_batch"])["limn_commit_batch"]
+        args = (ctypes.c_void_p * 2)(ctypes.c_void_p(dev_table.ptr), ctypes.c_void_p(len(commits)))
         params = (ctypes.c_void_p * 2)(*[ctypes.addressof(args) + k * ctypes.sizeof(ctypes.c_void_p) for k in range(2)])
-        check(self.api.hipModuleLaunchKernel(fn, len(entries), 1, 1, 256, 1, 1, 0, None, params, None), "launching the commits")
+        check(self.api.hipModuleLaunchKernel(self._commit_kernel, blocks, 1, 1, 256, 1, 1, 0, None, params, None), "launching the commits")
         self._committed += commits
 
     def finish(self) -> None:
