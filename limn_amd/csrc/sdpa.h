@@ -44,6 +44,11 @@ int launch_mfma_bwd(const SdpaArgs& a, void* ws, int passes);  // LIMN_HIP_BWD_*
 bool rows_supports(int dtype, int64_t hd, int64_t hd_v);
 int launch_sdpa_rows(SdpaPass pass, const SdpaArgs& a);
 
+// General-width forward calls on 16-bit matrix cores with split probabilities (sdpa_split.hip): f16 and
+// bf16, head dims in multiples of 8 up to 128, no causal mask. launch_sdpa_rows hands them over.
+bool split_takes(SdpaPass pass, const SdpaArgs& a);
+int launch_sdpa_split(const SdpaArgs& a);
+
 // The general-width calls whose float32 arithmetic runs on matrix cores (sdpa_wide.h): f32, f16 and
 // bf16, head dims in multiples of 4 up to 128, enough rows. launch_sdpa_rows hands them over.
 bool wide_takes(SdpaPass pass, const SdpaArgs& a);

@@ -434,6 +434,7 @@ bool wide_takes(SdpaPass pass, const SdpaArgs& a) {
 }
 
 int launch_sdpa_rows(SdpaPass pass, const SdpaArgs& a) {
+  if (split_takes(pass, a)) return launch_sdpa_split(a);
   if (wide_takes(pass, a))
     return a.dtype == LIMN_HIP_FLOAT32   ? launch_wide_f32(pass, a)
            : a.dtype == LIMN_HIP_FLOAT16 ? launch_wide_f16(pass, a)

@@ -148,3 +148,31 @@ def test_same_bits_twice(hipdev):
     a, b = (run(hipdev, "float32", *x, None, True, 0.2) for _ in range(2))
     for p, q in zip(a, b):
         np.testing.assert_array_equal(p, q)
+
+
+# (batch, t_q, t_k, hd, hd_v, masked): query and key tile edges (128, 64), each padded width, unequal dims
+SPLIT_CASES = [(20, 1, 64, 32, 32, False), (16, 129, 65, 16, 24, True), (3, 128, 63, 64, 40, True), (2, 130, 200, 96, 96, False),
+               (2, 40, 129, 80, 80, True), (1, 7, 1, 128, 104, False), (5, 64, 512, 120, 120, True)]
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=str)
+def test_split_probabilities_match_float64(hipdev, case, dtype):
+    """The non-causal half-width forward (csrc/sdpa_split.hip): one rounding at the store is all it adds."""
+    B, tq, tk, hd, hv, masked = case
+    rng = np.random.default_rng(tk)
+    q, k, v, do = (rng.standard_normal(s) for s in ((B, tq, hd), (B, tk, hd), (B, tk, hv), (B, tq, hv)))
+    mask = (rng.random((B, tk)) < 0.6).astype(np.float64) if masked else None
+    if masked:
+        mask[:, -1] = 1
+    want = exact(dtype, q, k, v, do, mask, False, hd**-0.5)
+    if masked:  # what a hidden key holds reaches nothing
+        k, v = np.where(mask[..., None] != 0, k, np.inf), np.where(mask[..., None] != 0, v, np.nan)
+    got = run(hipdev, dtype, q, k, v, do, mask, False, hd**-0.5)
+    rel = ROUND[dtype] / 2 + 1e-5  # half an ulp of the stored value
+    np.testing.assert_allclose(got[0], want[0], rtol=rel, atol=1e-5)
+    np.testing.assert_allclose(got[1], want[1], rtol=1e-5, atol=1e-5)
+    if masked:
+        mask[0] = 0  # a row with every key hidden: NaN, and lse -inf
+        got = run(hipdev, dtype, q, k, v, do, mask, False, hd**-0.5)
+        assert np.isnan(got[0][0]).all() and np.isneginf(got[1][0]).all() and np.isfinite(got[0][1:]).all()
