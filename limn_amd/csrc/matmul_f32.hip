@@ -9,10 +9,9 @@
 // bytes needs 4-byte alignment only, and the buffer's range check is per dword, so a chunk that
 // straddles an operand's end reads its valid part and zeros.
 //
-// Tiles: 128 x 128 (4 waves of 64 x 64) when that alone gives every CU two workgroups, else 64 x 64
-// (4 waves of 32 x 32), four workgroups to a CU, with k split into slices while the tiles are too
-// few; the slices' partial tiles go to a workspace and are added per element in slice order, so
-// results do not depend on scheduling. k advances 32 per stage through two LDS buffers, one
+// Tiles: 128 x 128 (4 waves of 64 x 64) or 64 x 64 (4 waves of 32 x 32), see plan_f32, with k split
+// into slices while the tiles are too few; the slices' partial tiles go to a workspace and are added
+// per element in slice order, so results do not depend on scheduling. k advances 32 per stage through two LDS buffers, one
 // barrier per stage, the next stage's loads in flight under the current one's products.
 //
 // LDS tiles keep their memory orientation. k-contiguous: [rows][32 + 4], a lane takes the four k
@@ -21,20 +20,30 @@
 // Row-contiguous: [32][rows + 8], the same k values by four ds_read_b32, the two 32-lane halves
 // four LDS rows and so half the banks apart.
 //
-// Accuracy: a running total is rounded once per product, so its error grows with the square root
-// of its length; every FOLD stages (256 k) the accumulators are added to a second set and
-// cleared, which keeps a sum over thousands of rows (a weight gradient) as close to the exact one
-// as the 64 interleaved partial sums of the general reduce kernel this replaced.
+// Accuracy: the product adds its terms one after another, each sum rounded, so a running total's error
+// grows with the square root of its length; every two stages (64 k) the accumulators are added to a
+// second set and start again from zero. Where the general reduce kernels hold many partial sums (an
+// operand contiguous along k, or few cells) the 64 also go in four chains of 16, at some 5% of the time;
+// where those kernels add all of k in one thread (a weight gradient) in one. Off float64, relative to the
+// result, general kernels / these: x @ w^T at k = 512 1.0e-7/1.0e-7, 2048 1.3e-7/1.1e-7; x^T @ y over 256
+// rows 2.9e-7/1.5e-7, over 2048 8.1e-7/1.6e-7.
 //
 // Measured figures are at f32_pays and plan_f32 below.
+
+#include <type_traits>
 
 #include "matmul.h"
 
 namespace limn {
+
+// Four chains a cell where the general kernels sum as closely (see the accuracy note).
+static bool f32_chains(const MatmulShape& s) {
+  return s.a_k == 1 || s.b_k == 1 || s.batch * s.M * s.N < ((int64_t)1 << 18);
+}
+
 namespace {
 
 constexpr int FB = 32;    // k per stage
-constexpr int FOLD = 8;   // stages between folds of the accumulators into the totals
 constexpr int FTHREADS = 256;
 
 template <int ROWS, bool KCONTIG>
@@ -103,8 +112,8 @@ __device__ __forceinline__ float f32_terms(float v, int relu, const MatmulAddend
   return v;
 }
 
-template <int BT, bool A_K, bool B_K, bool PARTIAL>
-__global__ __launch_bounds__(FTHREADS, BT == 128 ? 2 : 4) void matmul_f32(const float* __restrict__ a, const float* __restrict__ b,
+template <int BT, int CH, bool A_K, bool B_K, bool PARTIAL>
+__global__ __launch_bounds__(FTHREADS, BT == 128 ? 2 : CH == 4 ? 3 : 4) void matmul_f32(const float* __restrict__ a, const float* __restrict__ b,
                                                                           float* __restrict__ c, MatmulShape s, int64_t chunk,
                                                                           int wide, int relu, MatmulAddends add) {
   constexpr int T = BT / 64;  // 32 x 32 accumulators per wave along m and along n
@@ -131,13 +140,13 @@ __global__ __launch_bounds__(FTHREADS, BT == 128 ? 2 : 4) void matmul_f32(const 
   const int64_t m0 = tm * BT, n0 = tn * BT;
   const int k_lo = (int)(slice * chunk), depth = (int)(slice * chunk + chunk < s.K ? slice * chunk + chunk : s.K);
 
-  f32x16 acc[T][T], total[T][T];
+  f32x16 acc[CH][T][T], total[T][T];
 #pragma unroll
   for (int i = 0; i < T; i++)
 #pragma unroll
     for (int j = 0; j < T; j++)
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] = total[i][j][e] = 0.f;
+      for (int e = 0; e < 16; e++) total[i][j][e] = 0.f;
 
   OA oa(a + bz * s.a_batch, s.M, s.K, A_K ? s.a_m : s.a_k, m0);
   OB ob(b + bz * s.b_batch, s.N, s.K, B_K ? s.b_n : s.b_k, n0);
@@ -151,9 +160,11 @@ __global__ __launch_bounds__(FTHREADS, BT == 128 ? 2 : 4) void matmul_f32(const 
   oa.store(As[0]);
   ob.store(Bs[0]);
   __syncthreads();
-  for (int st = 0; st < stages; st++) {
-    const float* at = As[st & 1];
-    const float* bt = Bs[st & 1];
+  // one stage from LDS buffer `cur` while the next is loaded, then stored to the other; `fresh` starts
+  // the accumulators from zero (as the product's constant third operand)
+  auto stage = [&](auto fresh, int st, int cur) __attribute__((always_inline)) {
+    const float* at = As[cur];
+    const float* bt = Bs[cur];
     const int next = k_lo + (st + 1) * FB;
     if (st + 1 < stages) {
       oa.load(next, depth);
@@ -172,17 +183,14 @@ __global__ __launch_bounds__(FTHREADS, BT == 128 ? 2 : 4) void matmul_f32(const 
 #pragma unroll
         for (int i = 0; i < T; i++)
 #pragma unroll
-          for (int j = 0; j < T; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[j][q], av[i][q], acc[i][j], 0, 0, 0);
-    }
-    if (st % FOLD == FOLD - 1) {
+          for (int j = 0; j < T; j++) {
+            f32x16& c = acc[q % CH][i][j];
+            f32x16 from = c;
+            if (decltype(fresh)::value && g == 0 && q < CH) {
 #pragma unroll
-      for (int i = 0; i < T; i++)
-#pragma unroll
-        for (int j = 0; j < T; j++)
-#pragma unroll
-          for (int e = 0; e < 16; e++) {
-            total[i][j][e] += acc[i][j][e];
-            acc[i][j][e] = 0.f;
+              for (int e = 0; e < 16; e++) from[e] = 0.f;
+            }
+            c = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[j][q], av[i][q], from, 0, 0, 0);
           }
     }
     if (st + 1 < stages) {
@@ -190,10 +198,21 @@ __global__ __launch_bounds__(FTHREADS, BT == 128 ? 2 : 4) void matmul_f32(const 
         oa.clear_tail(next, depth);
         ob.clear_tail(next, depth);
       }
-      oa.store(As[(st + 1) & 1]);
-      ob.store(Bs[(st + 1) & 1]);
+      oa.store(As[cur ^ 1]);
+      ob.store(Bs[cur ^ 1]);
     }
     __syncthreads();
+  };
+  for (int st = 0; st < stages; st += 2) {
+    stage(std::true_type{}, st, 0);
+    if (st + 1 < stages) stage(std::false_type{}, st + 1, 1);
+#pragma unroll
+    for (int i = 0; i < T; i++)
+#pragma unroll
+      for (int j = 0; j < T; j++)
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+          total[i][j][e] += CH == 4 ? (acc[0][i][j][e] + acc[1 % CH][i][j][e]) + (acc[2 % CH][i][j][e] + acc[3 % CH][i][j][e]) : acc[0][i][j][e];
   }
 
   // lane holds C[m = wm + 32 i + n32][n = wn + 32 j + 8 q + 4 h + e], e = 0..3
@@ -209,7 +228,7 @@ __global__ __launch_bounds__(FTHREADS, BT == 128 ? 2 : 4) void matmul_f32(const 
         if (col >= s.N) continue;
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = total[i][j][4 * q + e] + acc[i][j][4 * q + e];
+        for (int e = 0; e < 4; e++) v[e] = total[i][j][4 * q + e];
         float* o = PARTIAL ? c + ((slice * s.batch + bz) * s.M + row) * s.N + col : c + bz * s.c_batch + row * s.c_m + col * s.c_n;
         if (!PARTIAL) {
 #pragma unroll
@@ -239,25 +258,27 @@ __global__ __launch_bounds__(256) void matmul_f32_splits(const float* __restrict
   }
 }
 
-#define LIMN_F32_INSTANCE(BT, AK, BKC, P)                                                                             \
-  template __global__ void matmul_f32<BT, AK, BKC, P>(const float* __restrict__, const float* __restrict__, float* __restrict__, \
-                                                      MatmulShape, int64_t, int, int, MatmulAddends);
-#define LIMN_F32_LAYOUT(BT, P) \
-  LIMN_F32_INSTANCE(BT, true, true, P) LIMN_F32_INSTANCE(BT, true, false, P) LIMN_F32_INSTANCE(BT, false, true, P) LIMN_F32_INSTANCE(BT, false, false, P)
-LIMN_F32_LAYOUT(128, false)
-LIMN_F32_LAYOUT(64, false)
-LIMN_F32_LAYOUT(64, true)
+#define LIMN_F32_INSTANCE(BT, CH, AK, BKC, P)                                                                             \
+  template __global__ void matmul_f32<BT, CH, AK, BKC, P>(const float* __restrict__, const float* __restrict__, float* __restrict__, \
+                                                          MatmulShape, int64_t, int, int, MatmulAddends);
+#define LIMN_F32_LAYOUT(BT, CH, P) \
+  LIMN_F32_INSTANCE(BT, CH, true, true, P) LIMN_F32_INSTANCE(BT, CH, true, false, P) LIMN_F32_INSTANCE(BT, CH, false, true, P) LIMN_F32_INSTANCE(BT, CH, false, false, P)
+LIMN_F32_LAYOUT(128, 1, false)
+LIMN_F32_LAYOUT(64, 1, false)
+LIMN_F32_LAYOUT(64, 1, true)
+LIMN_F32_LAYOUT(64, 4, false)
+LIMN_F32_LAYOUT(64, 4, true)
 #undef LIMN_F32_LAYOUT
 #undef LIMN_F32_INSTANCE
 
-template <int BT, bool A_K, bool B_K, bool PARTIAL>
+template <int BT, int CH, bool A_K, bool B_K, bool PARTIAL>
 int launch_tiles(const float* a, const float* b, float* c, const MatmulShape& s, const MatmulPlan& plan, int relu,
                  const MatmulAddends& add, hipStream_t stream) {
   const int64_t blocks = plan.split * s.batch * ((s.M + BT - 1) / BT) * ((s.N + BT - 1) / BT);
   if (blocks > 0x7fffffff) return fail(LIMN_HIP_EUNSUPPORTED, "contract: %lld workgroups exceed one launch", (long long)blocks);
   const bool rows16 = s.c_n == 1 && s.c_m % 4 == 0 && s.c_batch % 4 == 0;
   const int wide = (uintptr_t)c % 16 == 0 && (PARTIAL ? s.N % 4 == 0 : rows16);
-  hipLaunchKernelGGL((matmul_f32<BT, A_K, B_K, PARTIAL>), dim3((unsigned)blocks), dim3(FTHREADS), 0, stream, a, b, c, s,
+  hipLaunchKernelGGL((matmul_f32<BT, CH, A_K, B_K, PARTIAL>), dim3((unsigned)blocks), dim3(FTHREADS), 0, stream, a, b, c, s,
                      plan.chunk, wide, relu, add);
   return check_hip(hipGetLastError(), "launching the float32 contraction");
 }
@@ -265,10 +286,13 @@ int launch_tiles(const float* a, const float* b, float* c, const MatmulShape& s,
 template <bool A_K, bool B_K>
 int launch_layout(const float* a, const float* b, float* c, const MatmulShape& s, const MatmulPlan& plan, int relu,
                   const MatmulAddends& add, float* ws, hipStream_t stream) {
+  if (plan.tile == 128) return launch_tiles<128, 1, A_K, B_K, false>(a, b, c, s, plan, relu, add, stream);
+  const bool chains = f32_chains(s);
   if (plan.split == 1)
-    return plan.tile == 128 ? launch_tiles<128, A_K, B_K, false>(a, b, c, s, plan, relu, add, stream)
-                            : launch_tiles<64, A_K, B_K, false>(a, b, c, s, plan, relu, add, stream);
-  const int rc = launch_tiles<64, A_K, B_K, true>(a, b, ws, s, plan, relu, add, stream);
+    return chains ? launch_tiles<64, 4, A_K, B_K, false>(a, b, c, s, plan, relu, add, stream)
+                  : launch_tiles<64, 1, A_K, B_K, false>(a, b, c, s, plan, relu, add, stream);
+  const int rc = chains ? launch_tiles<64, 4, A_K, B_K, true>(a, b, ws, s, plan, relu, add, stream)
+                        : launch_tiles<64, 1, A_K, B_K, true>(a, b, ws, s, plan, relu, add, stream);
   if (rc != LIMN_HIP_OK) return rc;
   const int64_t total = s.batch * s.M * s.N;
   const int64_t blocks = (total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096;
@@ -299,17 +323,16 @@ bool f32_pays(const MatmulShape& s) {
   return (double)s.batch * (double)s.M * (double)s.N * (double)s.K >= (double)((int64_t)1 << 23);
 }
 
-// 128 x 128 tiles when there are two for every CU; else 64 x 64, four to a CU. Those too few to give
-// every CU two cut k: into slices of at least 512 up to four workgroups a CU, or, where slices that
-// long cannot give every CU two, into slices of at least 128 that do. Measured, us (TFLOP/s), the
-// general kernels before: (4096 x 512 -> 2048) 88 (98), 7000 before; (4096 x 2048 -> 512) 91 (94),
-// its weight gradient over 4096 rows, four slices, 86 (100), 91 with two; 1024^3 two slices 31 (68),
-// four 37; 2048^3 unsplit 64 x 64 152 (113), 4096^3 1053 (130; the matrix cores reach 154 in a
-// large library product).
+// One chain: 128 x 128 tiles when there are two for every CU. Else 64 x 64, four to a CU. Those too few
+// to give every CU two cut k: into slices of at least 512 up to four workgroups a CU, or, where slices
+// that long cannot give every CU two, into slices of at least 128 that do. Measured, us (TFLOP/s), the
+// general kernels before: (4096 x 512 -> 2048) 92 (93), 7000 before; (4096 x 2048 -> 512) 93 (92), its
+// weight gradient over 4096 rows, four slices, 84 (102), 91 with two; 1024^3 two slices 31 (68), four
+// 37; 2048^3 152 (113), 4096^3 x^T @ y 1080 (127; the matrix cores reach 154 in a large library product).
 MatmulPlan plan_f32(const MatmulShape& s) {
   const int64_t t128 = s.batch * ((s.M + 127) / 128) * ((s.N + 127) / 128);
   const int64_t t64 = s.batch * ((s.M + 63) / 64) * ((s.N + 63) / 64);
-  if (t128 >= 512) return {128, 1, s.K};
+  if (t128 >= 512 && !f32_chains(s)) return {128, 1, s.K};
   if (t64 >= 512) return {64, 1, s.K};
   int64_t split = 1024 / t64 < s.K / 512 ? 1024 / t64 : s.K / 512;
   if (split * t64 < 512) split = 512 / t64 < s.K / 128 ? 512 / t64 : s.K / 128;

@@ -1,8 +1,8 @@
 """limn_hip_contract, the float32 contraction, through the C ABI on the GPU and through plans of nests.
 
 Tolerance: a product and an addition of a float32 sum each round once (2^-24 of the value), a running
-total is at most 256 products long, then the 256-long totals and the k slices are added, so the error
-of a cell is under (256 + K / 256 + slices + 3) 2^-24 times its sum of |a b| (and the terms').
+total is at most 64 products long, then the 64-long totals and the k slices are added, so the error
+of a cell is under (64 + K / 64 + slices + 3) 2^-24 times its sum of |a b| (and the terms').
 """
 
 from __future__ import annotations
@@ -63,7 +63,7 @@ def test_contract_layouts(hipdev, a_kcontig, b_kcontig, M, N, K):
         if terms:
             want, bound = res + (want + bias), size + np.abs(bias) + np.abs(res)
         slices = 1 if not room else -(-need // (4 * batch * M * N))
-        assert (np.abs(got - want) <= (min(K, 256) + K / 256 + slices + 3) * 2.0**-24 * bound).all()
+        assert (np.abs(got - want) <= (min(K, 64) + K / 64 + slices + 3) * 2.0**-24 * bound).all()
 
 
 def test_contract_keeps_infinities_and_nans_to_their_rows(hipdev):
