@@ -172,22 +172,28 @@ int limn_hip_matmul_supported(int dtype, int64_t M, int64_t N, int64_t K, int64_
                               int64_t b_batch, int64_t b_k, int64_t b_n);
 
 /*
- * limn_hip_matmul_add for float32, limn's default type: float32 operands, products, totals, result,
- * bias and residual; one stride of each operand must be 1, the other any (no alignment past the
- * element's). Replaces the same reference kernel as limn_hip_matmul (limn/cuda_emit.py:376-685).
- * Same workspace rules, with limn_hip_contract_workspace(...) bytes.
+ * limn_hip_matmul_add for the contractions limn_hip_matmul refuses: float32 (limn's default type:
+ * float32 operands, products, totals, result, bias and residual), and bf16 / f16 with operand rows
+ * that are not 16-byte aligned or a k that is no multiple of 8 (copied to aligned rows in the
+ * workspace first). One stride of each operand must be 1, the other any. Replaces the same reference
+ * kernel as limn_hip_matmul (limn/cuda_emit.py:376-685). The workspace rules are limn_hip_matmul's for
+ * float32; a half width needs its limn_hip_contract_workspace(...) bytes.
  */
 int limn_hip_contract(const void* a, const void* b, void* c, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                       int64_t a_batch, int64_t a_m, int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int64_t c_batch,
                       int64_t c_m, int64_t c_n, int epilogue, const void* bias, int bias_dtype, int64_t bias_n,
                       const void* residual, int64_t r_batch, int64_t r_m, int64_t r_n, void* workspace,
                       int64_t workspace_bytes, void* stream);
-int64_t limn_hip_contract_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K);
 
-/* 1 when limn_hip_contract takes this layout and is the faster way to compute it (a very small
- * contraction is left to the general reduce kernels), else 0. */
+/* 1 when limn_hip_contract takes this dtype and operand layout, else 0; and the workspace it uses. `shifted`:
+ * bit 0 when a does not start on a 16-byte boundary, bit 1 when b does not (float32 ignores it). */
 int limn_hip_contract_supported(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t a_batch, int64_t a_m,
-                                int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n);
+                                int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int shifted);
+int64_t limn_hip_contract_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t a_batch, int64_t a_m,
+                                    int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int shifted);
+
+/* 1 when it is also the faster way: a very small contraction is one launch of a general reduce kernel. */
+int limn_hip_contract_pays(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K);
 
 /*
  * A pre-bound launch list: the kernels of one recorded execution of a plan, replayed against new

@@ -254,7 +254,9 @@ int limn_hip_contract(const void* a, const void* b, void* c, int dtype, int64_t 
                       const void* residual, int64_t r_batch, int64_t r_m, int64_t r_n, void* workspace,
                       int64_t workspace_bytes, void* stream) {
   MatmulShape s = {batch, M, N, K, a_batch, a_m, a_k, b_batch, b_k, b_n, c_batch, c_m, c_n};
-  if (dtype != LIMN_HIP_FLOAT32) return fail(LIMN_HIP_EUNSUPPORTED, "contract: takes float32, not dtype code %d", dtype);
+  const bool half = dtype == LIMN_HIP_BFLOAT16 || dtype == LIMN_HIP_FLOAT16;
+  if (dtype != LIMN_HIP_FLOAT32 && !half)
+    return fail(LIMN_HIP_EUNSUPPORTED, "contract: takes float32, bfloat16 or float16, not dtype code %d", dtype);
   if (batch < 1 || M < 1 || N < 1 || K < 1)
     return fail(LIMN_HIP_EINVAL, "contract: sizes must be positive (batch %lld, M %lld, N %lld, K %lld)", (long long)batch,
                 (long long)M, (long long)N, (long long)K);
@@ -262,26 +264,46 @@ int limn_hip_contract(const void* a, const void* b, void* c, int dtype, int64_t 
   if (epilogue != MATMUL_EPILOGUE_NONE && epilogue != MATMUL_EPILOGUE_RELU)
     return fail(LIMN_HIP_EINVAL, "contract: unknown epilogue %d", epilogue);
   if (workspace_bytes < 0) return fail(LIMN_HIP_EINVAL, "contract: negative workspace size");
-  if (bias != nullptr && bias_dtype != dtype)
-    return fail(LIMN_HIP_EINVAL, "contract: the bias is of the output type, not dtype %d", bias_dtype);
-  if (!f32_layout_ok(s)) return fail(LIMN_HIP_EUNSUPPORTED, "contract: operands must be contiguous along m/n or k, within 2 GiB a batch entry");
-  if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)bias | (uintptr_t)residual) % 4 != 0)
+  if (bias != nullptr && bias_dtype != dtype && !(half && bias_dtype == LIMN_HIP_FLOAT32))
+    return fail(LIMN_HIP_EINVAL, "contract: the bias is of the output type (or float32 under a half width), not dtype %d", bias_dtype);
+  const uintptr_t size = half ? 2 : 4;
+  const int bias_f32 = bias != nullptr && bias_dtype == LIMN_HIP_FLOAT32;
+  if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)residual) % size != 0 || (uintptr_t)bias % (bias_f32 ? 4 : size) != 0)
     return fail(LIMN_HIP_EINVAL, "contract: buffers must be aligned to their element size");
-  MatmulAddends add = {bias, 1, bias_n, residual, r_batch, r_m, r_n, 0};
-  return launch_matmul_f32(a, b, c, s, epilogue, add, workspace, workspace_bytes, (hipStream_t)stream);
+  MatmulAddends add = {bias, bias_f32, bias_n, residual, r_batch, r_m, r_n, 0};
+  if (!half) {
+    if (!f32_layout_ok(s)) return fail(LIMN_HIP_EUNSUPPORTED, "contract: operands must be contiguous along m/n or k, within 2 GiB a batch entry");
+    return launch_matmul_f32(a, b, c, s, epilogue, add, workspace, workspace_bytes, (hipStream_t)stream);
+  }
+  const bool a_shifted = (uintptr_t)a % 16 != 0, b_shifted = (uintptr_t)b % 16 != 0;
+  if (!pack_layout_ok(s, a_shifted, b_shifted))
+    return fail(LIMN_HIP_EUNSUPPORTED, "contract: operands must be contiguous along m/n or k, within 2 GiB a batch entry");
+  if (workspace == nullptr || (uintptr_t)workspace % 16 != 0 || workspace_bytes < pack_workspace_bytes(s, a_shifted, b_shifted))
+    return fail(LIMN_HIP_EINVAL, "contract: a half-width contraction needs its workspace, 16-byte aligned");
+  if (bias != nullptr && bias_n == 1 && (uintptr_t)bias % 16 == 0) add.vec |= 1;
+  if (residual != nullptr && r_n == 1 && r_m % 8 == 0 && r_batch % 8 == 0 && (uintptr_t)residual % 16 == 0) add.vec |= 2;
+  return launch_matmul_packed(a, b, c, dtype, s, epilogue, add, workspace, (hipStream_t)stream);
 }
 
-int64_t limn_hip_contract_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K) {
-  if (dtype != LIMN_HIP_FLOAT32 || batch < 1 || M < 1 || N < 1 || K < 1) return 0;
-  MatmulShape s = {batch, M, N, K, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  return f32_workspace_bytes(s);
+int64_t limn_hip_contract_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t a_batch, int64_t a_m,
+                                    int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int shifted) {
+  if (!limn_hip_contract_supported(dtype, batch, M, N, K, a_batch, a_m, a_k, b_batch, b_k, b_n, shifted)) return 0;
+  MatmulShape s = {batch, M, N, K, a_batch, a_m, a_k, b_batch, b_k, b_n, 0, 0, 0};
+  return dtype == LIMN_HIP_FLOAT32 ? f32_workspace_bytes(s) : pack_workspace_bytes(s, shifted & 1, shifted & 2);
 }
 
 int limn_hip_contract_supported(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t a_batch, int64_t a_m,
-                                int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n) {
-  if (dtype != LIMN_HIP_FLOAT32 || batch < 1 || M < 1 || N < 1 || K < 1) return 0;
+                                int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int shifted) {
+  if (batch < 1 || M < 1 || N < 1 || K < 1) return 0;
   MatmulShape s = {batch, M, N, K, a_batch, a_m, a_k, b_batch, b_k, b_n, 0, 0, 0};
-  return f32_layout_ok(s) && f32_pays(s);
+  if (dtype == LIMN_HIP_FLOAT32) return f32_layout_ok(s);
+  return (dtype == LIMN_HIP_BFLOAT16 || dtype == LIMN_HIP_FLOAT16) && pack_layout_ok(s, shifted & 1, shifted & 2);
+}
+
+int limn_hip_contract_pays(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K) {
+  const double products = (double)batch * (double)M * (double)N * (double)K;
+  if (dtype == LIMN_HIP_FLOAT32) return products >= F32_PAYS;
+  return products >= PACK_PAYS && M >= PACK_SIDE && N >= PACK_SIDE && K >= PACK_SIDE;
 }
 
 int64_t limn_hip_matmul_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K) {

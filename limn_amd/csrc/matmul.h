@@ -41,12 +41,30 @@ int matmul_layout_ok(const MatmulShape& s);
 int launch_matmul(const void* a, const void* b, void* c, int dtype, const MatmulShape& s, int epilogue,
                   const MatmulAddends& add, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
+// Products from which limn_hip_contract beats the general reduce kernels, whose one launch may also be
+// merged with its neighbours. One call, us, general / contract (x @ w^T; x @ w; x^T @ y):
+// float32: (64 x 784 -> 128) 5.5/9.9, 8.3/10.0, 8.5/10.5; (32 x 512 -> 512) 16.2/8.9, 8.4/9.3, 8.4/9.3;
+// (256 x 256 -> 256) 30.1/8.8, 43.5/8.8, 8.5/9.3; 512^3 224/11, 334/11, 40/12; 1024^3 1771/31, 3113/31,
+// 260/31. Half widths pay for the copies: 257^3 14/15, 22/15, 9/15; 321^3 22/14, 75/14,
+// 14/15; (65 x 8193 -> 65) 16/22, 130/21, 17/21; (129 x 4097 -> 129) 28/21, 251/21, 26/21; 513^3 68/18,
+// 297/19, 46/19; 1025^3 651/29, 2697/30, 280/29. With a side under 64 the copy, padded to whole stages of
+// 64, and the idle part of a tile can outweigh the product: (2^18 x 33 -> 33) 159/59, 123/59, 131/58, but
+// (2^19 x 9 -> 9) 24/100, 28/99, 16/93 and (33 x 2^18 -> 33) 60/77, 862/103, 132/106.
+constexpr double F32_PAYS = 1 << 23, PACK_PAYS = 1 << 26;
+constexpr int64_t PACK_SIDE = 64;
+
 // float32 operands and result (matmul_f32.hip), any row stride and alignment.
 bool f32_layout_ok(const MatmulShape& s);
-bool f32_pays(const MatmulShape& s);  // faster than the general reduce kernels
 MatmulPlan plan_f32(const MatmulShape& s);
 int64_t f32_workspace_bytes(const MatmulShape& s);
 int launch_matmul_f32(const void* a, const void* b, void* c, MatmulShape s, int epilogue, const MatmulAddends& add,
                       void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
+// Half widths with any row alignment and any k, through aligned copies of the operands that need them
+// (matmul_pack.hip). `shifted`: the operand does not start on a 16-byte boundary.
+bool pack_layout_ok(const MatmulShape& s, bool a_shifted, bool b_shifted);
+int64_t pack_workspace_bytes(const MatmulShape& s, bool a_shifted, bool b_shifted);
+int launch_matmul_packed(const void* a, const void* b, void* c, int dtype, const MatmulShape& s, int epilogue,
+                         const MatmulAddends& add, void* workspace, hipStream_t stream);
 
 }  // namespace limn

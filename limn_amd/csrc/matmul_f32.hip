@@ -28,7 +28,7 @@
 // result, general kernels / these: x @ w^T at k = 512 1.0e-7/1.0e-7, 2048 1.3e-7/1.1e-7; x^T @ y over 256
 // rows 2.9e-7/1.5e-7, over 2048 8.1e-7/1.6e-7.
 //
-// Measured figures are at f32_pays and plan_f32 below.
+// Measured figures are at plan_f32 below and at F32_PAYS (matmul.h).
 
 #include <type_traits>
 
@@ -312,15 +312,6 @@ bool f32_layout_ok(const MatmulShape& s) {
            ((double)(rows + 128) * row_stride + (double)(depth + 2 * FB) * k_stride + 256) * 4 < (double)INT32_MAX;
   };
   return reach(s.M, s.K, s.a_m, s.a_k) && reach(s.N, s.K, s.b_n, s.b_k);
-}
-
-// Below 2^23 products the general reduce kernels' one launch (which may also be merged with its
-// neighbours) is as fast as a product and its slice fold. One call, us, general / this (x @ W^T;
-// x @ W; x^T @ y): (64 x 784 -> 128) 5.5/9.9, 8.3/10.0, 8.5/10.5; (32 x 512 -> 512) 16.2/8.9,
-// 8.4/9.3, 8.4/9.3; (256 x 256 -> 256) 30.1/8.8, 43.5/8.8, 8.5/9.3; 512^3 224/11, 334/11, 40/12;
-// 1024^3 1771/40, 3113/39, 260/38.
-bool f32_pays(const MatmulShape& s) {
-  return (double)s.batch * (double)s.M * (double)s.N * (double)s.K >= (double)((int64_t)1 << 23);
 }
 
 // One chain: 128 x 128 tiles when there are two for every CU. Else 64 x 64, four to a CU. Those too few

@@ -477,18 +477,31 @@ def read_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
     return con
 
 
-def contraction_supported(con: Contraction) -> bool:
-    """Whether liblimn_hip.so takes this contraction: the half widths with 16-byte aligned operand
-    rows (limn_hip_matmul), float32 with any (limn_hip_contract)."""
+def takes_matmul(con: Contraction) -> bool:
+    """Whether limn_hip_matmul takes this contraction: a half width with 16-byte aligned operand rows."""
     from limn_amd.dtypes import ABI_CODE
 
-    lib, code = runtime.kernels(), ABI_CODE[con.dtype]
-    strides = (con.a_batch, con.a_m, con.a_k, con.b_batch, con.b_k, con.b_n)
-    if con.dtype is float32:
-        return bool(lib.limn_hip_contract_supported(code, con.batch, con.M, con.N, con.K, *strides))
-    if con.a_offset % 8 or con.b_offset % 8:
+    if con.dtype is float32 or con.a_offset % 8 or con.b_offset % 8:
         return False
-    return bool(lib.limn_hip_matmul_supported(code, con.M, con.N, con.K, *strides))
+    return bool(runtime.kernels().limn_hip_matmul_supported(ABI_CODE[con.dtype], con.M, con.N, con.K, con.a_batch, con.a_m, con.a_k,
+                                                            con.b_batch, con.b_k, con.b_n))
+
+
+def contract_sizes(con: Contraction) -> tuple:
+    """The arguments of limn_hip_contract_supported and limn_hip_contract_workspace."""
+    from limn_amd.dtypes import ABI_CODE
+
+    shifted = (con.a_offset * con.dtype.itemsize % 16 != 0) + 2 * (con.b_offset * con.dtype.itemsize % 16 != 0)
+    return (ABI_CODE[con.dtype], con.batch, con.M, con.N, con.K, con.a_batch, con.a_m, con.a_k, con.b_batch, con.b_k, con.b_n, shifted)
+
+
+def contraction_supported(con: Contraction) -> bool:
+    """Whether liblimn_hip.so takes this contraction, through limn_hip_matmul or (float32, unaligned
+    half-width rows) limn_hip_contract, where that is faster than the general reduce kernels."""
+    if takes_matmul(con):
+        return True
+    lib, sizes = runtime.kernels(), contract_sizes(con)
+    return bool(lib.limn_hip_contract_pays(*sizes[:5]) and lib.limn_hip_contract_supported(*sizes))
 
 
 def _vec_width(nest_shape: NestShape, bufs: Buffers, var: str, extent: int) -> int:
@@ -2754,18 +2767,18 @@ def _keep_runner(producer_inputs: dict, k: int):
 
 def _matmul_launcher(dev, con: Contraction, epilogue: int, adds: bool = False):
     """launch(inputs, out_ptr, bias_ptr, residual_ptr): the contraction through limn_hip_matmul, or
-    through limn_hip_matmul_add when `adds` (the residual read at the output's strides); a float32
-    one through limn_hip_contract either way."""
+    through limn_hip_matmul_add when `adds` (the residual read at the output's strides); one that
+    neither takes through limn_hip_contract either way."""
     from limn_amd.dtypes import ABI_CODE
 
     lib = dev.lib
     code = ABI_CODE[con.dtype]
     size = con.dtype.itemsize
     shape = (code, con.batch, con.M, con.N, con.K, con.a_batch, con.a_m, con.a_k, con.b_batch, con.b_k, con.b_n, con.c_batch, con.c_m, con.c_n, epilogue)
-    wide = con.dtype is float32
-    entry, step = (lib.limn_hip_contract, replay.STEP_CONTRACT) if wide else (lib.limn_hip_matmul_add, replay.STEP_MATMUL_ADD)
-    workspace = lib.limn_hip_contract_workspace if wide else lib.limn_hip_matmul_workspace
-    ws_bytes = int(workspace(code, con.batch, con.M, con.N, con.K))
+    general = not takes_matmul(con)
+    entry, step = (lib.limn_hip_contract, replay.STEP_CONTRACT) if general else (lib.limn_hip_matmul_add, replay.STEP_MATMUL_ADD)
+    ws_bytes = int(lib.limn_hip_contract_workspace(*contract_sizes(con)) if general
+                   else lib.limn_hip_matmul_workspace(code, con.batch, con.M, con.N, con.K))
     held: list = []  # the split-k workspace, allocated on first use and kept with the runner
 
     def launch(inputs: list, out: int, bias: int | None = None, res: int | None = None, bias_code: int = code) -> None:
@@ -2774,7 +2787,7 @@ def _matmul_launcher(dev, con: Contraction, epilogue: int, adds: bool = False):
         a = inputs[con.a_input].ptr + con.a_offset * size
         b = inputs[con.b_input].ptr + con.b_offset * size
         ws = held[0].ptr if held else None
-        if adds or wide:
+        if adds or general:
             args = (a, b, out, *shape, bias, bias_code, 1, res, con.c_batch, con.c_m, con.c_n, ws, ws_bytes)
             runtime.check_limn(entry(*args, None))
             if dev.tape is not None:

@@ -85,8 +85,9 @@ _LIMN = {
                             + [c_int, c_void_p, c_int, _I64, c_void_p, _I64, _I64, _I64, c_void_p, _I64, c_void_p]),
     "limn_hip_contract": (c_int, [c_void_p, c_void_p, c_void_p, c_int] + [_I64] * 13
                           + [c_int, c_void_p, c_int, _I64, c_void_p, _I64, _I64, _I64, c_void_p, _I64, c_void_p]),
-    "limn_hip_contract_workspace": (_I64, [c_int, _I64, _I64, _I64, _I64]),
-    "limn_hip_contract_supported": (c_int, [c_int] + [_I64] * 10),
+    "limn_hip_contract_workspace": (_I64, [c_int] + [_I64] * 10 + [c_int]),
+    "limn_hip_contract_supported": (c_int, [c_int] + [_I64] * 10 + [c_int]),
+    "limn_hip_contract_pays": (c_int, [c_int] + [_I64] * 4),
     "limn_hip_matmul_workspace": (_I64, [c_int, _I64, _I64, _I64, _I64]),
     "limn_hip_replay": (c_int, [c_void_p, _I64, c_void_p, _I64, c_void_p, _I64, c_void_p]),
     "limn_hip_replay_graph": (c_int, [c_void_p, _I64, c_void_p, _I64, c_void_p, _I64, c_void_p]),

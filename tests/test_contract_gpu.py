@@ -1,6 +1,6 @@
-"""limn_hip_contract, the float32 contraction, through the C ABI on the GPU and through plans of nests.
+"""limn_hip_contract, the contraction of float32 and of unaligned half widths, through the C ABI on the GPU and through plans of nests.
 
-Tolerance: a product and an addition of a float32 sum each round once (2^-24 of the value), a running
+Tolerance in float32: a product and an addition of a sum each round once (2^-24 of the value), a running
 total is at most 64 products long, then the 64-long totals and the k slices are added, so the error
 of a cell is under (64 + K / 64 + slices + 3) 2^-24 times its sum of |a b| (and the terms').
 """
@@ -44,7 +44,7 @@ def test_contract_layouts(hipdev, a_kcontig, b_kcontig, M, N, K):
     keep_res, pres = upload(hipdev, res, odd)
     (a_m, a_k), (b_k, b_n) = ((K, 1) if a_kcontig else (1, M)), ((1, K) if b_kcontig else (N, 1))
     lib = hipdev.lib
-    need = lib.limn_hip_contract_workspace(F32, batch, M, N, K)
+    need = lib.limn_hip_contract_workspace(F32, batch, M, N, K, M * K, a_m, a_k, K * N, b_k, b_n, 0)
     ws = hipdev.alloc(max(need, 4))
     total = a.astype(np.float64) @ b.astype(np.float64)
     size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
@@ -102,8 +102,58 @@ def test_contract_refuses_what_it_cannot_run(hipdev):
     def call(dtype=F32, K=4, a_m=4, a_k=1, bias_dtype=F32, c=p, ws=0):
         return lib.limn_hip_contract(p, p, c, dtype, 1, 4, 4, K, 0, a_m, a_k, 0, 4, 1, 0, 4, 1, 0, p, bias_dtype, 1, None, 0, 0, 0, None, ws, None)
 
-    assert [call(dtype=3), call(a_m=8, a_k=2), call(a_m=1 << 30)] == [2, 2, 2]
-    assert [call(K=0), call(bias_dtype=3), call(c=p + 2), call(ws=-1)] == [1, 1, 1, 1]
+    assert [call(dtype=0), call(a_m=8, a_k=2), call(a_m=1 << 30)] == [2, 2, 2]
+    assert [call(K=0), call(bias_dtype=3), call(c=p + 2), call(ws=-1), call(dtype=3, bias_dtype=3)] == [1, 1, 1, 1, 1]
+
+
+# (a-k, b-k): each layout at one element, odd sizes, a k of whole 8s beside ragged rows, k tails about a
+# stage (64), rows wider than a tile, a split k
+HALF_SHAPES = [(1, 1, 1), (7, 9, 64), (65, 63, 65), (130, 127, 136), (33, 257, 63), (40, 24, 4099), (300, 517, 129)]
+
+
+@pytest.mark.parametrize("layout", [(1, 1), (1, 0), (0, 1), (0, 0)], ids=["kk", "kn", "mk", "mn"])
+@pytest.mark.parametrize("M,N,K", HALF_SHAPES, ids=str)
+def test_contract_half_widths_any_alignment(hipdev, layout, M, N, K):
+    """Whole numbers up to 8 in float16: every product and float32 total is exact, so the result is the
+    float64 one rounded to float16, then rounded again with the terms added (limn_hip_matmul_add's
+    rule). The operands sit between NaNs, half of them off a 16-byte boundary."""
+    rng = np.random.default_rng(M + N + K)
+    half, batch, lib = 2, 2, hipdev.lib
+    shift = [(M + K) % 2, (N // 8) % 2 * 3]
+
+    def put(x, off):
+        flat = np.concatenate([np.full(off, np.nan), x.reshape(-1), np.full(9, np.nan)]).astype(np.float16)
+        buf = hipdev.alloc(flat.nbytes)
+        hipdev.copyin(buf, flat)
+        return buf, buf.ptr + 2 * off
+
+    a, b = (rng.integers(-8, 9, (batch, *d)).astype(np.float64) for d in ((M, K), (K, N)))
+    bias, res = rng.integers(-8, 9, N).astype(np.float64), rng.integers(-8, 9, (batch, M, N)).astype(np.float64)
+    a[0, 0, 0] = np.inf  # stays in its row
+    b[1, K - 1, N - 1] = np.nan  # and this in its column
+    keep_a, pa = put(a if layout[0] else a.swapaxes(1, 2), shift[0])
+    keep_b, pb = put(b.swapaxes(1, 2) if layout[1] else b, shift[1])
+    keep_bias, pbias = put(bias, 1)
+    keep_res, pres = put(res, 1)
+    keep_c, pc = put(np.full(batch * M * N, 7.0), 1)
+    (a_m, a_k), (b_k, b_n) = ((K, 1) if layout[0] else (1, M)), ((1, K) if layout[1] else (N, 1))
+    sizes = (half, batch, M, N, K, M * K, a_m, a_k, K * N, b_k, b_n)
+    shifted = (pa % 16 != 0) + 2 * (pb % 16 != 0)
+    assert lib.limn_hip_contract_supported(*sizes, shifted)
+    need = lib.limn_hip_contract_workspace(*sizes, shifted)
+    ws = hipdev.alloc(max(need, 16))
+    hipdev.copyin(ws, np.full(max(need, 16) // 4, np.nan, np.float32))
+    call = (pa, pb, pc, *sizes, M * N, N, 1, 0, pbias, half, 1, pres, M * N, N, 1, ws.ptr)
+    if need:
+        assert lib.limn_hip_contract(*call, need - 1, None) == 1
+    runtime.check_limn(lib.limn_hip_contract(*call, need, None))
+    hipdev.finish()
+    got = hipdev.copyout(keep_c).view(np.float16)
+    assert np.isnan(got[1 + batch * M * N :]).all() and np.isnan(got[0])
+    with np.errstate(invalid="ignore"):
+        total = (a @ b).astype(np.float16).astype(np.float64)
+        want = (res + (total + bias)).astype(np.float16)
+    np.testing.assert_array_equal(got[1 : 1 + batch * M * N].reshape(batch, M, N), want)
 
 
 @pytest.mark.parametrize("lead", [(512,), (4, 128)], ids=["rows", "batched"])

@@ -1,11 +1,11 @@
-"""Which float32 sums of products a plan hands to the matrix cores (no GPU)."""
+"""Which sums of products a plan hands to the matrix cores beyond the aligned half widths (no GPU)."""
 
 from __future__ import annotations
 
 import numpy as np
 import pytest
 
-from limn_amd.seam import Op, Tensor, custom, float32, grad, lower_all, realized, schedule, topological
+from limn_amd.seam import Op, Tensor, bfloat16, custom, float32, grad, lower_all, realized, schedule, topological
 from limn_amd.seam import device as limn_device
 
 emit = pytest.importorskip("limn_amd.hip.emit")
@@ -59,3 +59,13 @@ def test_a_mask_reaches_back_through_attention():
         nests = [n for n in lower_all(sinks, order, schedule(sinks, order))]
         sums = [n for n in nests if n.kernel.ast.op is Op.SUM]
         assert len(sums) == 1 and (realized(sums[0].kernel.target) in emit.deciding(nests)) is ordered
+
+
+@pytest.mark.parametrize("M,K,N,cores", [(513, 515, 517, True), (640, 1024, 129, True), (1023, 1031, 63, False), (300, 301, 303, False)], ids=str)
+def test_unaligned_half_width_sums(M, K, N, cores):
+    """Odd widths go to the copying contraction from 2^26 products, 64 of each side."""
+    a, b = (Tensor(rng.standard_normal(s).astype(np.float32), dtype=bfloat16) for s in ((M, K), (K, N)))
+    nests, kept = lowered([a @ b])
+    (con,) = [p.contraction for n, p in zip(nests, emit.plan_program(nests, kept, set()).plans) if n.kernel.ast.op is Op.SUM]
+    assert (con is not None) == cores
+    assert con is None or not emit.takes_matmul(con)
