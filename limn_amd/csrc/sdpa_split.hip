@@ -13,6 +13,14 @@
 // place. Dims between the width and the padded D are zeros in the tile. What bounds it is the softmax
 // arithmetic (exponentials, the split, the packing), which runs under the 16-bit products, as it does
 // not under float32 ones.
+//
+// An infinity in a live V row reaches every query that gives its key weight, but a split weight whose lo
+// part is zero or negative would make it NaN. A workgroup with a NaN in its totals, never one of finite
+// inputs, walks the keys once more with one small equal weight for each nonzero probability and no split,
+// and stores what comes out non-finite: the sign of an infinity, NaN where infinities meet or the
+// probability is 0.
+
+#include <type_traits>
 
 #include "sdpa_mfma.h"
 
@@ -85,92 +93,121 @@ __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restri
   for (int dt = 0; dt < D / 32; dt++) acc[dt] = zero16();
 
   const int ntiles = (t_k + TILE - 1) / TILE;
-  WidthStage<D> st;
-  st.template load<T, MASK>(krows, vrows, hd, hd_v, mrow, 0);
-  st.store(Ks[0], Vs[0]);
-  if (ntiles > 1) st.template load<T, MASK>(krows, vrows, hd, hd_v, mrow, TILE);
-  u16 mnext = MASK ? mrow.load(lane) : (u16)0;
-  __syncthreads();
-  for (int it = 0; it < ntiles; it++) {
-    const int k0 = it * TILE, buf = it & 1;
-    const u16* Kt = Ks[buf];
-    const u16* Vt = Vs[buf];
-    uint64_t live = ~0ull;
-    if (MASK) {
-      live = live_keys<T>(mnext);
-      if (it + 1 < ntiles) mnext = mrow.load(k0 + TILE + lane);
-    }
-    f32x16 s[2] = {zero16(), zero16()};
-#pragma unroll
-    for (int ds = 0; ds < D / 16; ds++)
-#pragma unroll
-      for (int sub = 0; sub < 2; sub++) s[sub] = T::mfma32(read_row<D>(Kt, sub * 32 + n, 2 * ds + h), qf[ds], s[sub]);
-    if (k0 + TILE > t_k || (MASK && live != ~0ull)) {
-#pragma unroll
-      for (int sub = 0; sub < 2; sub++) {
-        const unsigned mb = (unsigned)(live >> (sub * 32 + 4 * h));
-#pragma unroll
-        for (int i = 0; i < 16; i++) s[sub][i] = hidden<false, MASK>(k0, sub, i, h, t_k, row, mb) ? neg_inf() : s[sub][i];
+  __shared__ int broken;
+  if (threadIdx.x == 0) broken = 0;  // the first barrier of walk orders it
+  auto walk = [&](auto first) __attribute__((always_inline)) {
+    constexpr bool SPLIT = decltype(first)::value;
+    WidthStage<D> st;
+    st.template load<T, MASK>(krows, vrows, hd, hd_v, mrow, 0);
+    st.store(Ks[0], Vs[0]);
+    if (ntiles > 1) st.template load<T, MASK>(krows, vrows, hd, hd_v, mrow, TILE);
+    u16 mnext = MASK ? mrow.load(lane) : (u16)0;
+    __syncthreads();
+    for (int it = 0; it < ntiles; it++) {
+      const int k0 = it * TILE, buf = it & 1;
+      const u16* Kt = Ks[buf];
+      const u16* Vt = Vs[buf];
+      uint64_t live = ~0ull;
+      if (MASK) {
+        live = live_keys<T>(mnext);
+        if (it + 1 < ntiles) mnext = mrow.load(k0 + TILE + lane);
       }
-    }
-    float mx = neg_inf();
+      f32x16 s[2] = {zero16(), zero16()};
 #pragma unroll
-    for (int sub = 0; sub < 2; sub++)
+      for (int ds = 0; ds < D / 16; ds++)
 #pragma unroll
-      for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[sub][i]);
-    mx = pair_max(mx);
-    if (__any(mx > m + lift)) {  // the reference point moves as in sdpa_fwd_mfma
-      const float mnew = fmaxf(m, mx);
-      const float alpha = mnew == neg_inf() ? 1.f : fast_exp2((m - mnew) * c2);
-      l *= alpha;
+        for (int sub = 0; sub < 2; sub++) s[sub] = T::mfma32(read_row<D>(Kt, sub * 32 + n, 2 * ds + h), qf[ds], s[sub]);
+      if (k0 + TILE > t_k || (MASK && live != ~0ull)) {
 #pragma unroll
-      for (int dt = 0; dt < D / 32; dt++) acc[dt] *= alpha;
-      m = mnew;
-    }
-    const float base = m == neg_inf() ? 0.f : m * c2;
-    float rs = 0.f;
+        for (int sub = 0; sub < 2; sub++) {
+          const unsigned mb = (unsigned)(live >> (sub * 32 + 4 * h));
 #pragma unroll
-    for (int sub = 0; sub < 2; sub++)
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        s[sub][i] = fast_exp2(fmaf(s[sub][i], c2, -base));
-        rs += s[sub][i];
-      }
-    l += rs;
-#pragma unroll
-    for (int sub = 0; sub < 2; sub++)
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const u16x8 hi = pack8<T>(s[sub], 8 * c);
-        f32x16 rest;
-#pragma unroll
-        for (int e = 0; e < 8; e++) rest[e] = s[sub][8 * c + e] - T::unpack(hi[e]);
-        const u16x8 lo = pack8<T>(rest, 0);
-#pragma unroll
-        for (int dt = 0; dt < D / 32; dt++) {
-          const u16x8 vt = read_transposed<D>(Vt, sub * 32 + 16 * c, dt * 32);
-          acc[dt] = T::mfma32(vt, hi, acc[dt]);
-          acc[dt] = T::mfma32(vt, lo, acc[dt]);
+          for (int i = 0; i < 16; i++) s[sub][i] = hidden<false, MASK>(k0, sub, i, h, t_k, row, mb) ? neg_inf() : s[sub][i];
         }
       }
-    if (it + 1 < ntiles) {
-      st.store(Ks[buf ^ 1], Vs[buf ^ 1]);
-      if (it + 2 < ntiles) st.template load<T, MASK>(krows, vrows, hd, hd_v, mrow, k0 + 2 * TILE);
+      if constexpr (SPLIT) {
+        float mx = neg_inf();
+#pragma unroll
+        for (int sub = 0; sub < 2; sub++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[sub][i]);
+        mx = pair_max(mx);
+        if (__any(mx > m + lift)) {  // the reference point moves as in sdpa_fwd_mfma
+          const float mnew = fmaxf(m, mx);
+          const float alpha = mnew == neg_inf() ? 1.f : fast_exp2((m - mnew) * c2);
+          l *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < D / 32; dt++) acc[dt] *= alpha;
+          m = mnew;
+        }
+      }
+      const float base = m == neg_inf() ? 0.f : m * c2;
+      float rs = 0.f;
+#pragma unroll
+      for (int sub = 0; sub < 2; sub++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          s[sub][i] = fast_exp2(fmaf(s[sub][i], c2, -base));
+          rs += s[sub][i];
+          if constexpr (!SPLIT) s[sub][i] = s[sub][i] > 0.f ? 0x1p-14f : s[sub][i];
+        }
+      if constexpr (SPLIT) l += rs;
+#pragma unroll
+      for (int sub = 0; sub < 2; sub++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          const u16x8 hi = pack8<T>(s[sub], 8 * c);
+          f32x16 rest;
+#pragma unroll
+          for (int e = 0; e < 8; e++) rest[e] = s[sub][8 * c + e] - T::unpack(hi[e]);
+          const u16x8 lo = pack8<T>(rest, 0);
+#pragma unroll
+          for (int dt = 0; dt < D / 32; dt++) {
+            const u16x8 vt = read_transposed<D>(Vt, sub * 32 + 16 * c, dt * 32);
+            acc[dt] = T::mfma32(vt, hi, acc[dt]);
+            if constexpr (SPLIT) acc[dt] = T::mfma32(vt, lo, acc[dt]);
+          }
+        }
+      if (it + 1 < ntiles) {
+        st.store(Ks[buf ^ 1], Vs[buf ^ 1]);
+        if (it + 2 < ntiles) st.template load<T, MASK>(krows, vrows, hd, hd_v, mrow, k0 + 2 * TILE);
+      }
+      __syncthreads();
     }
-    __syncthreads();
-  }
+  };
+  walk(std::true_type{});
   const float total = pair_sum(l);
-  if (row >= t_q) return;
   const float mul = 1.f / total;
   u16* o = out + (b * (int64_t)t_q + row) * hd_v;
+  bool nan = false;
 #pragma unroll
   for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-      const int d = dt * 32 + 8 * g + 4 * h;
-      if (d < hd_v) *(u16x4*)(o + d) = u16x4{T::pack(acc[dt][4 * g] * mul), T::pack(acc[dt][4 * g + 1] * mul), T::pack(acc[dt][4 * g + 2] * mul), T::pack(acc[dt][4 * g + 3] * mul)};
+    for (int i = 0; i < 16; i++) nan |= acc[dt][i] != acc[dt][i];
+  if (nan && row < t_q) broken = 1;
+  if (row < t_q) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const int d = dt * 32 + 8 * g + 4 * h;
+        if (d < hd_v) *(u16x4*)(o + d) = u16x4{T::pack(acc[dt][4 * g] * mul), T::pack(acc[dt][4 * g + 1] * mul), T::pack(acc[dt][4 * g + 2] * mul), T::pack(acc[dt][4 * g + 3] * mul)};
     }
-  if (h == 0) lse[b * (int64_t)t_q + row] = m * scale + logf(total);
+    if (h == 0) lse[b * (int64_t)t_q + row] = m * scale + logf(total);
+  }
+  __syncthreads();
+  if (!broken) return;
+#pragma unroll
+  for (int dt = 0; dt < D / 32; dt++) acc[dt] = zero16();
+  walk(std::false_type{});
+  if (row >= t_q) return;
+#pragma unroll
+  for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int d = dt * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+      if (d < hd_v && !(fabsf(acc[dt][i]) < __builtin_inff())) o[d] = T::pack(acc[dt][i]);
+    }
 }
 
 template <typename T, int D>
@@ -203,7 +240,8 @@ int launch_split_width(const SdpaArgs& a) {
 // to 32 dims a few workgroups of 128 queries are no faster than waves that share out the keys: 1 head
 // 64 x 4096 x 32 63/67, 4 heads 33 x 77 x 32 6.1/6.8.
 bool split_takes(SdpaPass pass, const SdpaArgs& a) {
-  if (pass != SDPA_FWD || a.causal || !(a.scale > 0)) return false;
+  if (pass != SDPA_FWD || a.causal) return false;
+  if (!(a.scale >= 0x1p-64 && a.scale <= 0x1p64)) return false;  // scale log2(e) and its inverse, as floats, neither 0 nor infinite
   if (a.dtype != LIMN_HIP_FLOAT16 && a.dtype != LIMN_HIP_BFLOAT16) return false;
   if (a.hd % 8 != 0 || a.hd_v % 8 != 0 || a.hd > 128 || a.hd_v > 128) return false;
   const int64_t width = a.hd > a.hd_v ? a.hd : a.hd_v, rows = a.t_q > a.t_k ? a.t_q : a.t_k;

@@ -1506,11 +1506,10 @@ def deciding(nests: list[LoopNest]) -> set[Node]:
 
 
 def plan_nest(nest: LoopNest, inlined: "InlineSet | None" = None, stream: bool = False, ordered: bool = False) -> Planned:
-    """One nest's plan; `ordered` keeps a float32 sum of products on the general reduce kernels (see
-    `deciding`)."""
     """How one nest runs. With `inlined`, loads of the outputs of the producers it names are
     evaluated in place (see inline_producers); `stream` makes an elementwise nest's stores
-    non-temporal (see streamed_outputs)."""
+    non-temporal (see streamed_outputs); `ordered` keeps a float32 sum of products on the general
+    reduce kernels (see deciding)."""
     kernel = nest.kernel
     dtypes = {f"in{k}": n.dtype for k, n in enumerate(kernel.inputs)}
     dtypes["out"] = kernel.target.dtype

@@ -176,3 +176,27 @@ def test_split_probabilities_match_float64(hipdev, case, dtype):
         mask[0] = 0  # a row with every key hidden: NaN, and lse -inf
         got = run(hipdev, dtype, q, k, v, do, mask, False, hd**-0.5)
         assert np.isnan(got[0][0]).all() and np.isneginf(got[1][0]).all() and np.isfinite(got[0][1:]).all()
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("case", [(16, 129, 65, 32, 24, True), (3, 128, 63, 64, 40, False), (2, 40, 200, 128, 104, True)], ids=str)
+def test_split_probabilities_carry_an_infinity(hipdev, case, dtype):
+    """An infinity in a live value row reaches its dim of every query with its sign, also at weights that
+    16 bits hold exactly (no remainder) or round to zero; two that meet make NaN; other dims and other
+    heads keep their bits."""
+    B, tq, tk, hd, hv, masked = case
+    rng = np.random.default_rng(tk)
+    q, k, v, do = (rng.standard_normal(s) for s in ((B, tq, hd), (B, tk, hd), (B, tk, hv), (B, tq, hv)))
+    q[0, 1] = 0  # every weight 1
+    q[0, 2] = 8 * k[0, 0] / np.abs(k[0, 0]).max()  # most weights tiny
+    scale = hd**-0.5
+    mask = np.ones((B, tk)) if masked else None
+    if masked:
+        mask[:, 7:20] = 0
+    clean = run(hipdev, dtype, q, k, v, do, mask, False, scale)
+    v[0, 40, 3], v[0, 41, 9], v[0, [5, 50], 17] = np.inf, -np.inf, [np.inf, -np.inf]
+    got = run(hipdev, dtype, q, k, v, do, mask, False, scale)
+    assert np.isposinf(got[0][0, :, 3]).all() and np.isneginf(got[0][0, :, 9]).all() and np.isnan(got[0][0, :, 17]).all()
+    np.testing.assert_array_equal(np.delete(got[0][0], [3, 9, 17], axis=1), np.delete(clean[0][0], [3, 9, 17], axis=1))
+    np.testing.assert_array_equal(got[0][1:], clean[0][1:])
+    np.testing.assert_array_equal(got[1], clean[1])
