@@ -55,8 +55,9 @@ int limn_hip_device_info(int device, char* arch, int arch_len, int* compute_unit
                          int64_t* global_mem);
 
 /* Which kernel family serves an sdpa call of this shape: 1 = MFMA flash kernels, 0 = the
- * general-width kernels (any float dtype, any head dims up to 256; 64-bit or 32-bit arithmetic
- * throughout, the latter on matrix cores where the call is large enough), -1 = none. */
+ * general-width kernels (any float dtype, any head dims up to 256; scores, probabilities and totals
+ * of 64 or 32 bits, the latter on matrix cores where the call is large enough, and in 16-bit parts
+ * that add up to the float32 probabilities in the half widths' non-causal forward), -1 = none. */
 int limn_hip_sdpa_path(int dtype, int64_t hd, int64_t hd_v);
 
 /*

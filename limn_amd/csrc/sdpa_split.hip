@@ -1,12 +1,20 @@
 // Forward attention for f16 and bf16 at head dims the 16-bit family (sdpa_mfma.h) has no kernel for
 // (any multiple of 8 up to 128, hd and hd_v may differ), without a causal mask: 16-bit matrix products
-// with the probabilities kept to float32's worth of bits.
+// with the float32 probabilities split into 16-bit parts.
 //
 // S = Q K^T has 16-bit operands as they are stored, so its products are exact either way. P is float32
-// in the general-width kernels this takes calls over from; here it is split as P = hi + lo, each 16
-// bits (22 bits of P for f16, 16 for bf16), and O += hi V + lo V. What is left out is 2^-22 or 2^-17 of
-// each term, under the rounding of the output to its 11 or 8 bits: against float64, f16 256 heads 197 x 1021
-// x 80 is 2.1e-4 off with either kernel.
+// in the general-width kernels this takes calls over from; here it is a sum of 16-bit parts:
+//   bf16: three, each the rounding of what the ones before it leave. They hold all 24 bits of P; two left
+//     2^-19.5 of the terms' spread in an output whose terms cancel, where float32 leaves 2^-22.5.
+//   f16: hi + 2^-12 lo, the lo products in totals of their own. 11 + 11 bits and a sign, so at most the last
+//     bit of P is lost. f16 ends at 2^-24, so P carries a factor 2^SHIFT that its sum carries too: hi
+//     reaches 2^15, the top of the range, when a row's reference point lags by its LAG, and so does lo. A
+//     weight then loses at most 2^-49 of its row's largest (SHIFT + 12 + 25 bits down), a row less
+//     than 2^-49 times its keys times the largest value, which f16 can show (2^-25) only past 2^24.
+//     With no factor and hi and lo in one total a weight 2^-25 below the largest was dropped: a key of weight
+//     1 and value 0 among 1020 others 17 nats below it left an output 20% off.
+// Measured, us, two parts in one total / these: f16, 256 heads 197 x 1021 x 80, key mask, 57.0/57.3, 16 x 4096 x
+// 4096 x 80 172/174, 64 x 1024 x 1024 x 120 60/64 (the second totals spill there); bf16 56.6/62.3, 166/198, 58/68.
 //
 // The structure is sdpa_fwd_mfma's: 128 queries a workgroup, 32 a wave, 64-key tiles staged through
 // LDS a tile ahead, one lane per query row, the probability accumulators feeding the next product in
@@ -14,11 +22,11 @@
 // arithmetic (exponentials, the split, the packing), which runs under the 16-bit products, as it does
 // not under float32 ones.
 //
-// An infinity in a live V row reaches every query that gives its key weight, but a split weight whose lo
-// part is zero or negative would make it NaN. A workgroup with a NaN in its totals, never one of finite
-// inputs, walks the keys once more with one small equal weight for each nonzero probability and no split,
-// and stores what comes out non-finite: the sign of an infinity, NaN where infinities meet or the
-// probability is 0.
+// An infinity in a live V row reaches every query that gives its key weight, but a split weight with a part
+// that is zero or negative would make it NaN. A workgroup with a NaN in its totals (from a value that is
+// not finite, or a score that leaves float32) walks the keys once more with one small equal weight for
+// each nonzero probability and no split, and stores what comes out non-finite: the sign of an infinity,
+// NaN where infinities meet or the probability is 0 or NaN.
 
 #include <type_traits>
 
@@ -68,6 +76,42 @@ struct WidthStage {
   }
 };
 
+// How a storage type splits P (see above): 16-bit parts, sets of totals, log2 of P's factor and how far
+// (log2) a row's largest probability may pass its reference point.
+template <typename T>
+struct Split {  // bf16
+  static constexpr int PARTS = 3, TOTALS = 1;
+  static constexpr float SHIFT = 0.f, LAG = RESCALE_LOG2;
+};
+template <>
+struct Split<F16> {
+  static constexpr int PARTS = 2, TOTALS = 2;
+  static constexpr float SHIFT = 12.f, LAG = 3.f;
+};
+
+// Items base .. base + 7 of s as the parts of Split, most significant first.
+template <typename T>
+__device__ __forceinline__ void split8(const f32x16& s, int base, u16x8 (&part)[Split<T>::PARTS]) {
+  part[0] = pack8<T>(s, base);
+  if constexpr (Split<T>::TOTALS == 2) {
+    const f16x8 hi = __builtin_bit_cast(f16x8, part[0]);
+    f16x8 lo;
+#pragma unroll
+    for (int e = 0; e < 8; e++) lo[e] = (_Float16)fmaf((float)hi[e], -0x1p12f, s[base + e] * 0x1p12f);
+    part[1] = __builtin_bit_cast(u16x8, lo);
+  } else {
+    f32x16 rest;
+#pragma unroll
+    for (int e = 0; e < 8; e++) rest[e] = s[base + e];
+#pragma unroll
+    for (int p = 1; p < Split<T>::PARTS; p++) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) rest[e] -= T::unpack(part[p - 1][e]);
+      part[p] = pack8<T>(rest, 0);
+    }
+  }
+}
+
 template <typename T, int D, bool MASK>
 __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restrict__ q, const u16* __restrict__ k,
                                                              const u16* __restrict__ v, const u16* __restrict__ mask,
@@ -82,15 +126,21 @@ __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restri
   const Rows qrows(q + b * (int64_t)t_q * hd, t_q, hd);
   const Rows krows(k + b * (int64_t)t_k * hd, t_k, hd), vrows(v + b * (int64_t)t_k * hd_v, t_k, hd_v);
   const MaskRow mrow(MASK ? mask + b * (int64_t)t_k : nullptr, MASK ? t_k : 0);
-  const float c2 = scale * LOG2E, lift = RESCALE_LOG2 / c2;
+  typedef Split<T> P;
+  const float c2 = scale * LOG2E, lift = P::LAG / c2;
 
   u16x8 qf[D / 16];
-  f32x16 acc[D / 32];
+  f32x16 acc[P::TOTALS][D / 32];
   float m = neg_inf(), l = 0.f;
 #pragma unroll
   for (int ds = 0; ds < D / 16; ds++) qf[ds] = qrows.load8(ds * 16 + 8 * h < hd ? row * hd + ds * 16 + 8 * h : 0x3f000000);
+  auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int dt = 0; dt < D / 32; dt++) acc[dt] = zero16();
+    for (int t = 0; t < P::TOTALS; t++)
+#pragma unroll
+      for (int dt = 0; dt < D / 32; dt++) acc[t][dt] = zero16();
+  };
+  clear();
 
   const int ntiles = (t_k + TILE - 1) / TILE;
   __shared__ int broken;
@@ -137,11 +187,13 @@ __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restri
           const float alpha = mnew == neg_inf() ? 1.f : fast_exp2((m - mnew) * c2);
           l *= alpha;
 #pragma unroll
-          for (int dt = 0; dt < D / 32; dt++) acc[dt] *= alpha;
+          for (int t = 0; t < P::TOTALS; t++)
+#pragma unroll
+            for (int dt = 0; dt < D / 32; dt++) acc[t][dt] *= alpha;
           m = mnew;
         }
       }
-      const float base = m == neg_inf() ? 0.f : m * c2;
+      const float base = (m == neg_inf() ? 0.f : m * c2) - P::SHIFT;
       float rs = 0.f;
 #pragma unroll
       for (int sub = 0; sub < 2; sub++)
@@ -156,16 +208,13 @@ __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restri
       for (int sub = 0; sub < 2; sub++)
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-          const u16x8 hi = pack8<T>(s[sub], 8 * c);
-          f32x16 rest;
-#pragma unroll
-          for (int e = 0; e < 8; e++) rest[e] = s[sub][8 * c + e] - T::unpack(hi[e]);
-          const u16x8 lo = pack8<T>(rest, 0);
+          u16x8 part[P::PARTS];
+          split8<T>(s[sub], 8 * c, part);
 #pragma unroll
           for (int dt = 0; dt < D / 32; dt++) {
             const u16x8 vt = read_transposed<D>(Vt, sub * 32 + 16 * c, dt * 32);
-            acc[dt] = T::mfma32(vt, hi, acc[dt]);
-            if constexpr (SPLIT) acc[dt] = T::mfma32(vt, lo, acc[dt]);
+#pragma unroll
+            for (int p = 0; p < (SPLIT ? P::PARTS : 1); p++) acc[p % P::TOTALS][dt] = T::mfma32(vt, part[p], acc[p % P::TOTALS][dt]);
           }
         }
       if (it + 1 < ntiles) {
@@ -178,12 +227,18 @@ __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restri
   walk(std::true_type{});
   const float total = pair_sum(l);
   const float mul = 1.f / total;
+  if constexpr (P::TOTALS == 2) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[0][dt][i] = fmaf(acc[1][dt][i], 0x1p-12f, acc[0][dt][i]);
+  }
   u16* o = out + (b * (int64_t)t_q + row) * hd_v;
   bool nan = false;
 #pragma unroll
   for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
-    for (int i = 0; i < 16; i++) nan |= acc[dt][i] != acc[dt][i];
+    for (int i = 0; i < 16; i++) nan |= acc[0][dt][i] != acc[0][dt][i];
   if (nan && row < t_q) broken = 1;
   if (row < t_q) {
 #pragma unroll
@@ -191,14 +246,13 @@ __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restri
 #pragma unroll
       for (int g = 0; g < 4; g++) {
         const int d = dt * 32 + 8 * g + 4 * h;
-        if (d < hd_v) *(u16x4*)(o + d) = u16x4{T::pack(acc[dt][4 * g] * mul), T::pack(acc[dt][4 * g + 1] * mul), T::pack(acc[dt][4 * g + 2] * mul), T::pack(acc[dt][4 * g + 3] * mul)};
+        if (d < hd_v) *(u16x4*)(o + d) = u16x4{T::pack(acc[0][dt][4 * g] * mul), T::pack(acc[0][dt][4 * g + 1] * mul), T::pack(acc[0][dt][4 * g + 2] * mul), T::pack(acc[0][dt][4 * g + 3] * mul)};
     }
-    if (h == 0) lse[b * (int64_t)t_q + row] = m * scale + logf(total);
+    if (h == 0) lse[b * (int64_t)t_q + row] = m * scale + logf(total * __builtin_exp2f(-P::SHIFT));
   }
   __syncthreads();
   if (!broken) return;
-#pragma unroll
-  for (int dt = 0; dt < D / 32; dt++) acc[dt] = zero16();
+  clear();
   walk(std::false_type{});
   if (row >= t_q) return;
 #pragma unroll
@@ -206,7 +260,7 @@ __global__ __launch_bounds__(THREADS, 2) void sdpa_fwd_split(const u16* __restri
 #pragma unroll
     for (int i = 0; i < 16; i++) {
       const int d = dt * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-      if (d < hd_v && !(fabsf(acc[dt][i]) < __builtin_inff())) o[d] = T::pack(acc[dt][i]);
+      if (d < hd_v && !(fabsf(acc[0][dt][i]) < __builtin_inff())) o[d] = T::pack(acc[0][dt][i]);
     }
 }
 

@@ -200,3 +200,77 @@ def test_split_probabilities_carry_an_infinity(hipdev, case, dtype):
     np.testing.assert_array_equal(np.delete(got[0][0], [3, 9, 17], axis=1), np.delete(clean[0][0], [3, 9, 17], axis=1))
     np.testing.assert_array_equal(got[0][1:], clean[0][1:])
     np.testing.assert_array_equal(got[1], clean[1])
+
+
+def weighed(dtype, q, k, v, scale):
+    """The forward's output in float64; the sum of the sizes of its terms; the largest exponent (log2) of a weight."""
+    q, k, v = (stored(x, dtype)[1] for x in (q, k, v))
+    s = q @ k.swapaxes(1, 2) * scale
+    s -= s.max(-1, keepdims=True)
+    p = np.exp(s)
+    p /= p.sum(-1, keepdims=True)
+    return p @ v, p @ np.abs(v), -s.min() / np.log(2)
+
+
+def forward(dev, dtype, q, k, v, scale):
+    """(out, lse) of the device's forward."""
+    from limn_amd.dtypes import from_storage
+    from limn_amd import seam
+
+    t = getattr(seam, dtype)
+    B, tq, hd = q.shape
+    tk, hv = v.shape[1:]
+    bufs = []
+    for x in (q, k, v):
+        bits = stored(x, dtype)[0]
+        bufs.append(dev.alloc(bits.nbytes))
+        dev.copyin(bufs[-1], bits)
+    out, lse = dev.alloc(B * tq * hv * t.itemsize), dev.alloc(B * tq * 4)
+    runtime.check_limn(dev.lib.limn_hip_sdpa_fwd(*(b.ptr for b in bufs), None, out.ptr, lse.ptr, CODE[dtype], B, tq, tk, hd, hv, 0, scale, None))
+    dev.finish()
+    return from_storage(dev.copyout(out), t, (B, tq, hv)).astype(np.float64), dev.copyout(lse).view(np.float32).reshape(B, tq)
+
+
+def assert_float32_weights(got, want, size, far, dtype):
+    """A term of the sum in float32: its weight's exponent t = c s - c m carries the rounding of c (|t| 2^-24
+    of it) and its own, its score a few roundings, its product and additions a few more, (10 + 2 |t|) 2^-24
+    of the term in all. The store rounds once, in float16 to no less than 2^-25."""
+    step = ROUND[dtype] / 2
+    bound = step * np.abs(want) + (10 + 2 * far) * 2.0**-24 * size + (2.0**-25 if dtype == "float16" else 0.0)
+    worst = (np.abs(got - want) / bound).max()
+    assert worst <= 1, f"{worst:.2f} times the bound"
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("hd,hv", [(32, 32), (64, 40), (80, 80), (120, 120)], ids=str)
+def test_split_probabilities_hold_float32_weights(hipdev, hd, hv, dtype):
+    """Outputs whose terms cancel to 2^-15 of their spread, where the store's own rounding (2^-8 of them) is
+    under float32's: the terms' errors are then a few independent roundings, together some 2^-22.5 of
+    the spread in root mean square. Weights of 16 bits leave 2^-19.5."""
+    B, tq, tk = 3840 // hv, 1024, 48
+    rng = np.random.default_rng(hd)
+    q, k, v = (rng.standard_normal(s) for s in ((B, tq, hd), (B, tk, hd), (B, tk, hv)))
+    v *= 256
+    got = forward(hipdev, dtype, q, k, v, hd**-0.5)[0]
+    q, k, v = (stored(x, dtype)[1] for x in (q, k, v))
+    p = np.exp(q @ k.swapaxes(1, 2) * hd**-0.5)
+    p /= p.sum(-1, keepdims=True)
+    want, spread = p @ v, np.sqrt((p * p) @ (v * v))
+    near = np.abs(want) < 2.0**-15 * spread
+    assert near.sum() > 40
+    assert np.sqrt(np.mean(((got - want)[near] / spread[near]) ** 2)) < 2.0**-21
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("gap", [10, 14, 17, 20, 23])
+@pytest.mark.parametrize("case", [(16, 3, 1021, 32, 32), (2, 40, 4096, 80, 80), (2, 40, 1021, 96, 120)], ids=str)
+def test_split_probabilities_keep_small_weights(hipdev, case, gap, dtype):
+    """One key of weight near 1 and value zero among keys `gap` nats below it: the output is theirs alone,
+    and lse counts them too."""
+    B, tq, tk, hd, hv = case
+    rng = np.random.default_rng(tk + gap)
+    q, k = np.ones((B, tq, hd)), rng.standard_normal((B, tk, hd))
+    v = np.abs(rng.standard_normal((B, tk, hv))) * 1000
+    k[:, 300], v[:, 300] = gap * hd**-0.5, 0  # in a later tile than the first: the reference point moves to it
+    want, size, far = weighed(dtype, q, k, v, hd**-0.5)
+    assert_float32_weights(forward(hipdev, dtype, q, k, v, hd**-0.5)[0], want, size, far, dtype)
