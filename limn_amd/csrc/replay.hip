@@ -17,12 +17,6 @@ using namespace limn;
 
 namespace {
 
-// Lists this short are launched step by step also where a graph is asked for: a graph launch costs the
-// host some 25 us before its first kernel starts, while of a few launches the first starts at once
-// and the rest are issued under it. A captured call, graph / steps, us: 1 step (4096^3 product) 134/125,
-// 5 (float32 attention forward and backward) 90/80, 5 (bf16, 32 x 8 heads x 512) 143/127; 9 steps of
-// 2-5 us each 80/86, 86 steps 2045/2062. A new binding then needs no capture either.
-constexpr int64_t SHORT_LIST = 6;
 constexpr int MAX_ARGS = 512;  // a merged launch takes at most 400 pointers (the emitter's MERGE_PARAMS)
 
 // A zero fill as a kernel rather than hipMemsetAsync, so the list can be captured into a graph
@@ -246,7 +240,6 @@ extern "C" int limn_hip_replay_graph(const limn_hip_replay_step* steps, int64_t 
   if (rc != LIMN_HIP_OK) return rc;
   ReplayGraph* g = (ReplayGraph*)*handle;
   if (g == nullptr) *handle = g = new ReplayGraph();
-  if (nsteps <= SHORT_LIST) return run_list(steps, nsteps, args, slots, nullptr);
   if (!g->matches(steps, nsteps, args, nargs, slots, nslots)) {
     rc = g->capture(steps, nsteps, args, nargs, slots, nslots);
     if (rc != LIMN_HIP_OK) return rc;

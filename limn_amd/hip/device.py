@@ -145,7 +145,7 @@ class HipDevice(CompiledDevice):
         # run first, at most replay.PLANS_KEPT; `tape` collects the launches of the run that
         # records one (every launch site appends while it is set)
         self.replays: collections.OrderedDict[int, list] = collections.OrderedDict()
-        self.replay_graphs = True  # replay through a captured graph (False: launch by launch)
+        self.replay_graphs = True  # replay lists past replay.SHORT_LIST through a captured graph (False: launch by launch)
         self.tape: list[replay.Launch] | None = None
         self.issue_seconds = 0.0  # host time replayed runs spent before their barrier, summed
 
@@ -212,7 +212,7 @@ class HipDevice(CompiledDevice):
         one of three ways: a plan's first run call by call; its second also records every launch
         into a launch list (replay.py); later runs allocate fresh outputs, bind them and the
         sources to the list's slots and launch it in one native call, as a graph captured for
-        that binding unless `replay_graphs` is off. Results and commits are the same either way;
+        that binding unless `replay_graphs` is off or the list is short. Results and commits are the same either way;
         a recording whose buffers overlap is refused and the plan keeps running call by call."""
         entry = self.replays.get(id(plan))
         if entry is None or entry[0] is not plan:
@@ -307,7 +307,7 @@ class HipDevice(CompiledDevice):
             slots[prog.positions + i] = out.ptr
         for i, p in prog.out_positions:
             bufs[p] = outs[i]
-        check_limn(prog.run(self.lib, slots, self.finish, self.replay_graphs))
+        check_limn(prog.run(self.lib, slots, self.finish, self.replay_graphs and len(prog.steps) > replay.SHORT_LIST))
         for p, i in prog.assigns:
             self.commit(sources[p], outs[i])
             bufs[p] = outs[i]

@@ -12,7 +12,7 @@ one of the outputs the run allocated, in call order. A replay takes its outputs 
 the same few bindings recur run after run), binds every
 slot to this run's buffer and issues the whole list in one call: as a HIP graph captured for that
 binding (one capture serves every later run with the same buffers, and the launches cost the host
-one call), or launch by launch.
+one call), or launch by launch, as a list of at most SHORT_LIST steps always is.
 
 A recording is refused (the plan keeps running call by call) when two slots share bytes, since a
 pointer into them could not be told apart.
@@ -126,6 +126,10 @@ class Program:
         self.graphs.clear()
 
 
+# Lists this short are launched step by step also where graphs are on: a graph launch costs the host
+# some 25 us before its first kernel starts, while of a few launches the first starts at once and the
+# rest are issued under it. A new binding then needs no capture, and nothing is kept for one.
+SHORT_LIST = 6
 GRAPHS_PER_PLAN = 8
 PLANS_KEPT = 64  # launch lists a device keeps, the least recently run dropped first
 ARENAS_PER_PLAN = 3  # a list keeps this many output arenas; past that a replay takes a passing one

@@ -109,3 +109,73 @@ def test_the_device_keeps_a_bounded_number_of_launch_lists(monkeypatch):
         dev.run(p, {})
     assert list(dev.replays) == [id(plans[1]), id(plans[3]), id(plans[4])]
     assert lib.freed == 1  # the evicted list's graph was released
+
+
+class FakeHip:
+    """The runtime calls of a replay without host buffers or commits; counts the barriers."""
+
+    def __init__(self):
+        self.next_ptr, self.barriers = 0x10000, 0
+
+    def hipMalloc(self, ptr_ref, nbytes):
+        ptr_ref._obj.value = self.next_ptr
+        self.next_ptr += 0x10000
+        return 0
+
+    def hipDeviceSynchronize(self):
+        self.barriers += 1
+        return 0
+
+
+def replaying(lib) -> "tuple":
+    """A device over FakeHip, and a plan of one source and no outputs."""
+    from limn_amd.hip.device import HipDevice
+    from limn_amd.seam import Plan
+
+    dev = HipDevice.__new__(HipDevice)
+    dev.api, dev.lib, dev.pool = FakeHip(), lib, {}
+    dev._commits, dev._commit_targets, dev._committed = [], set(), []
+    dev.replay_graphs, dev.issue_seconds = True, 0.0
+    return dev, Plan(calls=(), buffers=(0,), sinks=(), positions=1)
+
+
+def steps_of(n: int) -> replay.Program:
+    steps, args = replay.bind([replay.Launch(replay.STEP_ZERO, (0x1000, 16))] * n, [(0, 0x1000, 16)])
+    return replay.Program(steps, args, (), (), (), 1)
+
+
+def test_a_short_list_captures_nothing_whatever_its_bindings():
+    """Past GRAPHS_PER_PLAN bindings a graph is dropped for each new one, behind a barrier; a list
+    launched step by step keeps nothing for a binding, so a run has its own barrier only."""
+    lib, prog = StubLib(graph_status=0), steps_of(replay.SHORT_LIST)
+    dev, plan = replaying(lib)
+    runs = replay.GRAPHS_PER_PLAN + 4
+    held = [dev._alloc(16) for _ in range(runs)]
+    for buf in held:
+        dev._replay(plan, prog, {0: buf})
+    assert (lib.graph_calls, lib.list_calls, prog.captures, len(prog.graphs)) == (0, runs, 0, 0)
+    assert dev.api.barriers == runs
+
+
+def test_a_list_past_the_short_ones_is_captured_per_binding():
+    lib, prog = StubLib(graph_status=0), steps_of(replay.SHORT_LIST + 1)
+    dev, plan = replaying(lib)
+    held = [dev._alloc(16), dev._alloc(16)]
+    for buf in held * 2:
+        dev._replay(plan, prog, {0: buf})
+    assert (lib.graph_calls, lib.list_calls, prog.captures, len(prog.graphs)) == (4, 0, 2, 2)
+
+
+def test_a_short_list_that_fails_is_not_run_again():
+    import pytest
+
+    class Failing(StubLib):
+        def limn_hip_replay(self, *args):
+            self.list_calls += 1
+            return 3
+
+    lib, prog = Failing(graph_status=3), steps_of(2)
+    dev, plan = replaying(lib)
+    with pytest.raises(RuntimeError):
+        dev._replay(plan, prog, {0: dev._alloc(16)})
+    assert (lib.graph_calls, lib.list_calls, prog.graph_failure) == (0, 1, None)
