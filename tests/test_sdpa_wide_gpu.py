@@ -274,3 +274,22 @@ def test_split_probabilities_keep_small_weights(hipdev, case, gap, dtype):
     k[:, 300], v[:, 300] = gap * hd**-0.5, 0  # in a later tile than the first: the reference point moves to it
     want, size, far = weighed(dtype, q, k, v, hd**-0.5)
     assert_float32_weights(forward(hipdev, dtype, q, k, v, hd**-0.5)[0], want, size, far, dtype)
+
+
+@pytest.mark.parametrize("dtype,size", [("float16", 2e3), ("float16", 1e4), ("bfloat16", 2e4), ("bfloat16", 3e6), ("bfloat16", 1e15)], ids=str)
+@pytest.mark.parametrize("hd,hv", [(32, 32), (80, 80), (96, 120)], ids=str)
+def test_split_probabilities_of_far_scores(hipdev, hd, hv, dtype, size):
+    """Scores of 10^7 to 10^31: a row is its nearest key's value row (the others are further below it
+    than its score's own rounding), and lse its score."""
+    B, tq, tk = 16, 40, 200
+    rng = np.random.default_rng(hd)
+    q, k, v = (rng.standard_normal(s) for s in ((B, tq, hd), (B, tk, hd), (B, tk, hv)))
+    q, k, v = (stored(x, dtype)[1] for x in (q * size, k * size, v))
+    k[:, 150] = k[:, 20]  # an equal score in a later tile
+    s = np.sort(q @ np.delete(k, 150, axis=1).swapaxes(1, 2), axis=-1) * hd**-0.5
+    clear = s[..., -1] - s[..., -2] > 40 + np.abs(s[..., -1]) * hd * 2.0**-23
+    assert clear.mean() > 0.9
+    want, _, _ = weighed(dtype, q, k, v, hd**-0.5)
+    out, lse = forward(hipdev, dtype, q, k, v, hd**-0.5)
+    np.testing.assert_allclose(out[clear], want[clear], rtol=ROUND[dtype] / 2 + 1e-5, atol=1e-5)
+    np.testing.assert_allclose(lse[clear], s[..., -1][clear], rtol=(hd + 2) * 2.0**-23)
