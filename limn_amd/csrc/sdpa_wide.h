@@ -73,6 +73,14 @@ __device__ __forceinline__ float wide_exp(float x) {
   return fast_exp2(t) * fmaf(lost, LN2, 1.f);
 }
 
+// s scale - L with the product rounded first, as in L itself: a row that one key dominates then has weight
+// 1, not e^(what the rounding of a far score took). At scores 64 times the usual spread dV was 5.0e-6 off
+// float64 without, 2.9e-6 with.
+__device__ __forceinline__ float wide_logit(float s, float scale, float L) {
+#pragma clang fp contract(off)
+  return s * scale - L;
+}
+
 template <typename T>
 __device__ __forceinline__ f32x4 wide_load4(__amdgpu_buffer_rsrc_t r, int off) {
   if constexpr (sizeof(typename T::Storage) == 4) {
@@ -123,18 +131,17 @@ struct WideRows {
   __device__ __forceinline__ float at(int row, int d) const { return wide_load1<T>(rsrc, d < width ? row * rb + d * SZ : FAR, 0); }
 };
 
-// the product of two row operands over all D dims: 32 dims at a time in chains that start from zero,
+// the product of two row operands over all D dims: SPAN dims at a time in chains that start from zero,
 // two chains, or one past 64 dims, where the registers of a second one spill (128 dims, 32 heads x 1024
-// rows, dK/dV: 494 us with two, 269 with two chains over all dims). Chains this short keep the scores as
-// close to float64's as the rows kernels' quarter rows do.
-template <int D>
-__device__ __forceinline__ f32x16 wide_scores(const f32x4 (&a)[D / 8], const f32x4 (&b)[D / 8]) {
+// rows, dK/dV: 494 us with two, 269 with two chains over all dims).
+template <int D, int SPAN>
+__device__ __forceinline__ f32x16 wide_dots(const f32x4 (&a)[D / 8], const f32x4 (&b)[D / 8]) {
   f32x16 s;
 #pragma unroll
-  for (int g0 = 0; g0 < D / 8; g0 += 4) {
+  for (int g0 = 0; g0 < D / 8; g0 += SPAN / 8) {
     f32x16 c0 = wide_zero(), c1 = wide_zero();
 #pragma unroll
-    for (int g = g0; g < g0 + 4; g++)
+    for (int g = g0; g < g0 + SPAN / 8; g++)
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         if (D > 64 || j % 2 == 0) c0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g][j], b[g][j], c0, 0, 0, 0);
@@ -147,6 +154,15 @@ __device__ __forceinline__ f32x16 wide_scores(const f32x4 (&a)[D / 8], const f32
     }
   }
   return s;
+}
+
+// Scores: their error counts in full in the exponential (and a row's sum of weights), so their chains are
+// as short as the rows kernels' quarter rows: 8 products at 32 dims, 16 past that. With twice that, outputs
+// of 24 heads x 512 rows x 32 dims, causal, were 1.46e-7 off float64 against the rows kernels' 1.37e-7, now
+// 1.36e-7; 96 dims 1.71e-7 against 1.55e-7, now 1.53e-7. It costs 0-4%.
+template <int D>
+__device__ __forceinline__ f32x16 wide_scores(const f32x4 (&a)[D / 8], const f32x4 (&b)[D / 8]) {
+  return wide_dots<D, D == 64 ? 32 : 16>(a, b);
 }
 
 // the 32-row sum of columns x probabilities, in two chains
@@ -406,7 +422,7 @@ __global__ __launch_bounds__(WTHREADS, D <= 32 ? 3 : D <= 64 ? 2 : 1) void sdpa_
     vm.rows(k0, vf);
     const unsigned live = wide_live<T>(mm, mask != nullptr, k0, t_k);
     f32x16 s = wide_scores<D>(kf, qf);
-    const f32x16 dp = wide_scores<D>(vf, of);
+    const f32x16 dp = wide_dots<D, 32>(vf, of);
     // a key that exists but is hidden has probability exp(-inf - L): zero, or NaN in a row whose
     // every key is hidden (L = -inf), as the numpy reference's; one past t_k or right of the row
     // is no term of the sum at all
@@ -486,7 +502,7 @@ __global__ __launch_bounds__(WTHREADS, D <= 32 ? 2 : 1) void sdpa_bwd_kv_wide(
       d4[g] = wide_load4<F32>(dm, (r0 + 8 * g + 4 * h) * 4);
     }
     f32x16 p = wide_scores<D>(qf, kf);
-    f32x16 ds = wide_scores<D>(of, vf);
+    f32x16 ds = wide_dots<D, D == 128 ? 16 : 32>(of, vf);  // at 128 dims the longer span spills: 16 x 2048 rows 1037 us, 897
     const bool edge = dead || r0 + WT > t_q || (causal && r0 < k0 + WT - 1);
     unsigned terms = ~0u;
     if (edge) {
@@ -503,7 +519,7 @@ __global__ __launch_bounds__(WTHREADS, D <= 32 ? 2 : 1) void sdpa_bwd_kv_wide(
     } else {
 #pragma unroll
       for (int i = 0; i < 16; i++) {
-        p[i] = wide_exp(fmaf(p[i], scale, -l4[i >> 2][i & 3]));
+        p[i] = wide_exp(wide_logit(p[i], scale, l4[i >> 2][i & 3]));
         ds[i] = p[i] * (ds[i] - d4[i >> 2][i & 3]) * scale;
       }
     }

@@ -293,3 +293,19 @@ def test_split_probabilities_of_far_scores(hipdev, hd, hv, dtype, size):
     out, lse = forward(hipdev, dtype, q, k, v, hd**-0.5)
     np.testing.assert_allclose(out[clear], want[clear], rtol=ROUND[dtype] / 2 + 1e-5, atol=1e-5)
     np.testing.assert_allclose(lse[clear], s[..., -1][clear], rtol=(hd + 2) * 2.0**-23)
+
+
+@pytest.mark.parametrize("hd", [24, 32, 48, 80, 96, 128])
+def test_a_far_score_keeps_its_whole_weight(hipdev, hd):
+    """Queries in line with one key, its score thousands above the others': a weight of exactly 1, whatever
+    the score's rounding, so dV is the plain sum of those queries' dO, and the output the key's row."""
+    B, tq, tk = 32, 200, 70
+    rng = np.random.default_rng(hd)
+    k, v, do = (rng.standard_normal(s).astype(np.float32) for s in ((B, tk, hd), (B, tk, hd), (B, tq, hd)))
+    k *= (8 / np.linalg.norm(k, axis=-1, keepdims=True)).astype(np.float32)
+    pick = rng.integers(0, tk, (B, tq))
+    q = 1234.5 * np.take_along_axis(k, pick[..., None], 1)
+    out, lse, _, _, dv = run(hipdev, "float32", q, k, v, do, None, False, 0.3)
+    np.testing.assert_array_equal(out, np.take_along_axis(v, pick[..., None], 1))
+    hot = (pick[..., None] == np.arange(tk)).astype(np.float64).swapaxes(1, 2)
+    assert (np.abs(dv - hot @ do) <= 16 * 2.0**-24 * (hot @ np.abs(do))).all()  # a key has some 3 queries, 10 at most
