@@ -193,7 +193,8 @@ int limn_hip_contract_supported(int dtype, int64_t batch, int64_t M, int64_t N, 
 int64_t limn_hip_contract_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t a_batch, int64_t a_m,
                                     int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int shifted);
 
-/* 1 when it is also the faster way: a very small contraction is one launch of a general reduce kernel. */
+/* 0 when a general reduce kernel (one launch) is the faster way whatever the layout: a very small
+ * contraction, a narrow one of a half width. A narrow float32 one of a long k may be as well. */
 int limn_hip_contract_pays(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K);
 
 /*

@@ -41,11 +41,11 @@ int matmul_layout_ok(const MatmulShape& s);
 int launch_matmul(const void* a, const void* b, void* c, int dtype, const MatmulShape& s, int epilogue,
                   const MatmulAddends& add, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
-// Products from which limn_hip_contract beats the general reduce kernels, whose one launch may also be
-// merged with its neighbours. One call, us, general / contract (x @ w^T; x @ w; x^T @ y):
-// float32: (64 x 784 -> 128) 5.5/9.9, 8.3/10.0, 8.5/10.5; (32 x 512 -> 512) 16.2/8.9, 8.4/9.3, 8.4/9.3;
-// (256 x 256 -> 256) 30.1/8.8, 43.5/8.8, 8.5/9.3; 512^3 224/11, 334/11, 40/12; 1024^3 1771/31, 3113/31,
-// 260/31. Half widths pay for the copies: 257^3 14/15, 22/15, 9/15; 321^3 22/14, 75/14,
+// Products below which the general reduce kernels, whose one launch may also be merged with its
+// neighbours, are never clearly the slower way. One call, us, general / contract (x @ w^T; x @ w; x^T @ y):
+// float32 from 2^23 on by layout and shape (emit.contract_pays): (64 x 784 -> 128) 4.3/9.8, 5.9/10.2, 5.8/10.7;
+// (32 x 512 -> 512) 16.4/8.4, 6.1/8.8, 5.6/9.2; (256 x 256 -> 256) 30.3/8.3, 43.7/8.6, 7.7/9.0; 512^3 226/11,
+// 334/11, 40/12; 1024^3 1771/31, 3113/31, 260/31. Half widths pay for the copies: 257^3 14/15, 22/15, 9/15; 321^3 22/14, 75/14,
 // 14/15; (65 x 8193 -> 65) 16/22, 130/21, 17/21; (129 x 4097 -> 129) 28/21, 251/21, 26/21; 513^3 68/18,
 // 297/19, 46/19; 1025^3 651/29, 2697/30, 280/29. With a side under 64 the copy, padded to whole stages of
 // 64, and the idle part of a tile can outweigh the product: (2^18 x 33 -> 33) 159/59, 123/59, 131/58, but

@@ -423,12 +423,6 @@ def _flat_reduce(inner: list[tuple[str, int]], ta: dict[str, int], tb: dict[str,
     return math.prod(extent.values()), ta[last], tb[last]
 
 
-def find_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
-    """The dense contraction a reduce nest is, when liblimn_hip.so takes it."""
-    con = read_contraction(nest, shape)
-    return con if con is not None and contraction_supported(con) else None
-
-
 def read_contraction(nest: LoopNest, shape: NestShape) -> Contraction | None:
     """The dense-contraction reading of a reduce nest (reference limn/cuda_emit.py:376-505
     detects the same shape, over one reduce var): a body of exactly two unmasked loads and their
@@ -497,11 +491,71 @@ def contract_sizes(con: Contraction) -> tuple:
 
 def contraction_supported(con: Contraction) -> bool:
     """Whether liblimn_hip.so takes this contraction, through limn_hip_matmul or (float32, unaligned
-    half-width rows) limn_hip_contract, where that is faster than the general reduce kernels."""
+    half-width rows) limn_hip_contract, where the sizes alone do not say that the general reduce
+    kernels are faster (for float32 see contract_pays)."""
     if takes_matmul(con):
         return True
     lib, sizes = runtime.kernels(), contract_sizes(con)
     return bool(lib.limn_hip_contract_pays(*sizes[:5]) and lib.limn_hip_contract_supported(*sizes))
+
+
+def contract_us(con: Contraction) -> float:
+    """Estimated time of a float32 limn_hip_contract call: 64 x 64 tiles, 32 of k a stage, 0.68 us a stage
+    for each round of 256 workgroups (a side under 64 idles part of its tiles) and 0.16 us of its
+    latency; then the fold, which adds a cell's k slices one after another. Within 25% of 94 in 100 of
+    1610 measured calls of 2^21 to 2^30 products, sides from 2 on."""
+    slices = 1
+    need = int(runtime.kernels().limn_hip_contract_workspace(*contract_sizes(con)))
+    cells = con.batch * con.M * con.N
+    if need:
+        slices = need // (4 * cells)
+    stages = -(-(-(-con.K // slices)) // 32)
+    groups = con.batch * -(-con.M // 64) * -(-con.N // 64) * slices
+    fold = 0.7 + 0.22 * slices + 1.2e-6 * need if need else 0.0
+    return 4.0 + 0.16 * stages + 0.68 * stages * max(1.0, groups / 256) + fold + 1.4e-6 * cells
+
+
+def general_us(con: Contraction, plan: Planned, across: bool) -> float:
+    """Estimated time of the same sum in the form plan_reduce chose for it; `across`: neighbouring
+    cells of the launch are not neighbours in memory. Rates, us a million products, from the same
+    calls: columns 0.17 + 0.25 / VEC; lanes along a contiguous k 0.15 + 0.55 / VEC, more where a row leaves
+    lanes idle, and 1.67 where k and n are both powers of two (as measured: 64 x 512, k 512 30.5 us, 100 x 320,
+    k 512 6.3); lanes along a k that one operand has strided 1.5; a thread a cell 0.26 to 0.35, or its stores."""
+    notes = plan.notes
+    millions = con.batch * con.M * con.N * con.K / 1e6
+    out_mb = 4e-6 * con.batch * con.M * con.N
+    in_mb = 4e-6 * con.K * ((con.batch if con.a_batch else 1) * con.M + (con.batch if con.b_batch else 1) * con.N)
+    rows = con.a_k == 1 and con.b_k == 1
+    vec = notes.get("vec", 1)
+    if "columns" in notes:
+        return 3.5 + millions * (0.17 + 0.25 / vec) + 0.2 * in_mb
+    lanes = notes.get("group", THREADS)
+    if lanes == 1:
+        if rows:
+            return 2.0 + 0.35 * millions + 0.2 * in_mb
+        if con.a_k == 1:
+            return 2.0 + 0.26 * millions + 0.15 * out_mb + 0.2 * in_mb
+        return 2.5 + max(0.3 * millions, (1.9 if across else 0.4) * out_mb)
+    if not rows:
+        return 3.5 + 1.5 * millions
+    if "parts" not in notes and con.K & (con.K - 1) == 0 and con.N & (con.N - 1) == 0:
+        return 2.5 + 1.67 * millions
+    chunks = con.K // vec
+    return 2.5 + millions * (0.39 * lanes / chunks if chunks < min(lanes, 64) else 0.15 + 0.55 / vec) + 0.1 * in_mb
+
+
+def contract_pays(con: Contraction, plan: Planned, across: bool) -> bool:
+    """Whether a float32 sum of products is faster through limn_hip_contract than in the general form
+    `plan`, by the estimates of both. The number of products alone does not tell: of 1297 measured calls
+    from 2^23 products on (x @ w^T, x @ w, x^T @ y and x^T @ w^T), 371 are faster in the general form,
+    narrow ones over a long k by up to 15 times. us, general / contract: x^T @ y of 10 x 784 over 4096 rows
+    10.4/18.0, 24 x 24 over 26080 8.8/44, 512 x 256 over 2048 50/20; x @ w^T 24 x 24, k 26080 7.0/43,
+    16 x 16, k 65536 7.7/113, 32 x 256, k 16384 223/41; x @ w 4 x 4096, k 4096 26.7/29.9, 256 x 256, k 256 43.7/8.6. By the
+    estimates 12 of them go the slower way by more than 5%, at most 1.48 times, and 52 stay general that
+    contract would run up to 1.74 times as fast. plan_tiled, which takes over from some general
+    forms, is not counted: up to 2^26 products it halves what x @ w^T still takes here (64 x 512, k 512
+    4.2/8.7)."""
+    return contract_us(con) < general_us(con, plan, across)
 
 
 def _vec_width(nest_shape: NestShape, bufs: Buffers, var: str, extent: int) -> int:
@@ -1521,9 +1575,15 @@ def plan_nest(nest: LoopNest, inlined: "InlineSet | None" = None, stream: bool =
     if shape.fold is None:
         return plan_elementwise(nest, shape, bufs, stream)
     con = read_contraction(nest, shape)
-    if con is not None and not (ordered and con.dtype is float32) and contraction_supported(con):
+    taken = con is not None and not (ordered and con.dtype is float32) and contraction_supported(con)
+    if taken and con.dtype is not float32:
         return Planned("", [], contraction=con, notes={"mfma": True})
     general = plan_reduce(nest, shape, bufs)
+    # once producers are evaluated in place the sum stays general, as its readers were planned
+    if taken and inlined is None:
+        across = bool(shape.outer) and dict(shape.out_index.terms).get(shape.outer[-1][0]) != 1
+        if contract_pays(con, general, across):
+            return Planned("", [], contraction=con, notes={"mfma": True})
     if con is not None and con.dtype is float32 and (inlined is None or not inlined.reached(nest)):
         return plan_tiled(nest, read_nest(nest), bufs, con, general) or general
     return general

@@ -5,7 +5,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from limn_amd.seam import Op, Tensor, bfloat16, custom, float32, grad, lower_all, realized, schedule, topological
+from limn_amd.seam import Node, Op, Tensor, bfloat16, custom, float32, grad, lower_all, realized, schedule, topological
 from limn_amd.seam import device as limn_device
 
 emit = pytest.importorskip("limn_amd.hip.emit")
@@ -27,7 +27,7 @@ def lowered(sinks: list[Tensor]):
 
 def float32_layer(train: bool, act) -> tuple[list, list]:
     """A float32 Linear, `act`, Linear: the plan's roles for its sums, forward only or trained."""
-    x = Tensor(rng.standard_normal((512, 256)).astype(np.float32), requires_grad=True)
+    x = Tensor(rng.standard_normal((2048, 256)).astype(np.float32), requires_grad=True)
     w1, w2 = (Tensor(rng.standard_normal(s).astype(np.float32), requires_grad=True) for s in ((256, 128), (128, 256)))
     y = act(x @ w1) @ w2
     sinks = [y, *grad((y * y).sum(), [x, w1, w2])] if train else [y]
@@ -69,3 +69,33 @@ def test_unaligned_half_width_sums(M, K, N, cores):
     (con,) = [p.contraction for n, p in zip(nests, emit.plan_program(nests, kept, set()).plans) if n.kernel.ast.op is Op.SUM]
     assert (con is not None) == cores
     assert con is None or not emit.takes_matmul(con)
+
+
+# (layout, M, N, K): each general form on both sides of its line; n is x @ w^T, w x @ w, g x^T @ y
+@pytest.mark.parametrize("layout,M,N,K,cores", [
+    ("g", 10, 784, 4096, False), ("g", 64, 512, 4096, True), ("g", 24, 24, 26080, False), ("g", 256, 256, 1024, True), ("g", 64, 64, 4096, False),
+    ("w", 2, 4096, 4096, False), ("w", 16, 4096, 4096, True), ("w", 64, 512, 512, False), ("w", 256, 256, 256, True), ("w", 2048, 2048, 2, False),
+    ("n", 16, 16, 65536, False), ("n", 24, 24, 26080, False), ("n", 512, 512, 512, True), ("n", 64, 512, 512, True), ("n", 300, 300, 784, True),
+], ids=str)
+def test_float32_sums_go_where_they_are_faster(layout, M, N, K, cores):
+    """Narrow sums, above all over a long k, stay on the general reduce kernels: measured, us, general /
+    contract: g 10 x 784 x 4096 10.4/18.0, 24 x 24 x 26080 8.8/44, 64 x 64 x 4096 7.3/16.8; w 2 x 4096 x 4096
+    20.3/29.7, 16 x 4096 x 4096 76/33, 64 x 512 x 512 7.3/9.1, 2048 x 2048 x 2 8.0/11.6; n 16 x 16 x 65536 7.7/113."""
+    def operand(*shape):
+        return Tensor.from_node(Node(Op.BUFFER, (), float32, shape, None))
+
+    if layout == "g":
+        out = operand(K, M).transpose() @ operand(K, N)
+    else:
+        out = operand(M, K) @ (operand(K, N) if layout == "w" else operand(N, K).transpose())
+    nests, kept = lowered([out])
+    (plan,) = [p for n, p in zip(nests, emit.plan_program(nests, kept, set()).plans) if n.kernel.ast.op is Op.SUM]
+    assert (plan.contraction is not None) == cores
+
+
+def test_a_declined_sum_keeps_its_epilogue_nests():
+    """A narrow sum that stays general runs its bias and relu readers as nests of their own."""
+    x, w = (Tensor.from_node(Node(Op.BUFFER, (), float32, s, None)) for s in ((65536, 24), (65536, 24)))
+    nests, kept = lowered([(x.transpose() @ w).relu()])
+    prog = emit.plan_program(nests, kept, set())
+    assert not prog.pairs and all(p.contraction is None for p in prog.plans)

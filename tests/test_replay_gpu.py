@@ -74,8 +74,8 @@ def attention(seed):
 def contract_float32(seed):
     """A float32 Linear long enough in k to be cut: partial tiles in a workspace, then the bias."""
     set_seed(seed)
-    layer = nn.Linear(2048, 130)
-    x = Tensor(np.random.default_rng(seed).standard_normal((96, 2048)).astype(np.float32))
+    layer = nn.Linear(2048, 260)
+    x = Tensor(np.random.default_rng(seed).standard_normal((300, 2048)).astype(np.float32))
     return [layer(x)]
 
 
@@ -119,7 +119,7 @@ def test_the_split_k_case_splits(hipdev):
     from limn_amd.dtypes import ABI_CODE
 
     assert hipdev.lib.limn_hip_matmul_workspace(ABI_CODE[bfloat16], 1, *SPLIT_K) > 0
-    assert hipdev.lib.limn_hip_contract_workspace(ABI_CODE[float32], 1, 96, 130, 2048, 0, 2048, 1, 0, 1, 2048, 0) > 0
+    assert hipdev.lib.limn_hip_contract_workspace(ABI_CODE[float32], 1, 300, 260, 2048, 0, 2048, 1, 0, 1, 2048, 0) > 0
 
 
 def results(dev, build, seed) -> list[np.ndarray]:
