@@ -57,7 +57,11 @@ int launch_wide_f16(SdpaPass pass, const SdpaArgs& a);
 int launch_wide_bf16(SdpaPass pass, const SdpaArgs& a);
 // 32-row blocks from which a wave walks its streamed rows alone; fewer are split in four (split, 256
 // heads x 512 rows x 64 dims, 4096 blocks: 133 us forward, 173 alone; 8192 x 32 x 32: equal).
+// One streamed tile of 32 rows leaves three of four waves nothing (2048 x 32 x 32 at 128 dims, dK/dV: 238 us split,
+// 175 alone, 190 on the rows kernels), and with two or three tiles a split pays only while blocks are few
+// (1024 x 64 at 16 dims, causal, 2048 blocks: 29/19/23; 64 x 64, 128 blocks: 7.2/9.6/6.1).
 constexpr int64_t WIDE_WAVES = 8192;
+constexpr int64_t WIDE_SHORT = 2048;  // the same with two or three streamed tiles
 // Workgroups of paired causal blocks from which blocks are paired (and 16 blocks a head); fewer leave
 // CUs idle and go a block each (8 heads x 256 rows: 12 us).
 constexpr int64_t WIDE_PAIRS = 512;

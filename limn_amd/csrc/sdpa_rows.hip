@@ -416,16 +416,26 @@ bool rows_supports(int dtype, int64_t hd, int64_t hd_v) {
 
 // Whether a call goes to the matrix-core kernels (sdpa_wide.h): what they can address, and enough
 // 32-row blocks that a wave each beats the lanes of the kernels above. One pass, us, rows / wide
-// (float32, causal; forward, dQ, dK/dV): 64 dims, 48 x 1024 rows at 32 dims 756/52, 912/66, 1140/98;
-// 8 heads x 128 rows of 64 13/9, 13/11, 13/13; 8 x 64 rows of 64 10.5/8.3, 10.7/9.8, 10.9/13.0;
-// 2 x 512 rows of 128 (32 blocks) 60/34, 66/48, 56/61; 32 x 64 rows of 128 27/16, 30/20, 31/28; 32 x 64
-// rows of 16 (64 blocks) 7.9/11.3, 5.1/5.9, 5.4/7.3, 128 x 64 of 16 10.0/9.3, 7.6/6.1, 8.5/7.5.
+// (float32; forward, dQ, dK/dV): 48 x 1024 rows at 32 dims, causal, 756/52, 912/66, 1140/98; 1 x 32 rows of 32 dims (one
+// block) 7.8/4.7, 8.1/4.6, 9.2/6.1; 16 x 64 rows of 64 10/7, 10/9, 11/12; 8 x 128 rows of 64 13/8, 14/10, 14/12; 1 x 1024
+// rows of 128 111/58, 124/85. A few blocks that stream one or two tiles (`tiles`) have the least to share out: 32 x 32 rows of 64
+// dims, causal, dK/dV 9.8/11.0, 128 x 32 19/11; 64 x 32 rows of 128 16/22, 128 x 32 30/22, and the forward and dQ of 16 x 64 rows
+// of 128 14/15, 16/20; 128 x 32 rows of 16 (128 blocks) 5.4/4.9, 4.9/5.5, 5.1/6.5, 512 x 32 7.4/5.2, 7.0/5.7, 7.5/6.8,
+// 64 x 64 of 16 6.6/5.5, 5.9/6.0, 6.1/7.2.
 bool wide_takes(SdpaPass pass, const SdpaArgs& a) {
   if (a.dtype == LIMN_HIP_FLOAT64 || a.hd % 4 != 0 || a.hd_v % 4 != 0 || a.hd > 128 || a.hd_v > 128) return false;
   if (a.t_q < 32 || a.t_k < 32) return false;  // a tile
+  const bool kv = pass == SDPA_BWD_KV;
   const int64_t width = a.hd > a.hd_v ? a.hd : a.hd_v;
-  const int64_t blocks = a.batch * (((pass == SDPA_BWD_KV ? a.t_k : a.t_q) + 31) / 32);
-  if (blocks < (width <= 16 ? 128 : width <= 32 ? 1 : width <= 64 || pass != SDPA_BWD_KV ? 32 : 64)) return false;
+  const int64_t blocks = a.batch * (((kv ? a.t_k : a.t_q) + 31) / 32), tiles = ((kv ? a.t_q : a.t_k) + 31) / 32;
+  int64_t least = 1;
+  if (width <= 16)
+    least = kv && tiles <= 2 ? 512 / tiles : pass == SDPA_BWD_Q && tiles == 1 ? 256 : 128;
+  else if (width > 32 && kv)
+    least = tiles == 1 && (width <= 64 || width > 96) ? 128 : width <= 64 && tiles > 2 ? 32 : 64;
+  else if (width > 32)
+    least = width > 96 && tiles <= 2 ? 64 : 32;
+  if (blocks < least) return false;
   // per-head byte offsets are 32-bit, below FAR and a tile past the end; loads are whole dwords
   const int64_t rows = a.t_q > a.t_k ? a.t_q : a.t_k;
   if ((rows + 256) * width * 4 >= (int64_t)0x70000000) return false;

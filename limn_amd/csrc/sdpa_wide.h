@@ -20,7 +20,7 @@
 //
 // A workgroup is four waves. KS = 4: one 32-row block, the waves taking streamed tiles w, w + 4, ...
 // and their totals combined at the end through LDS in wave order. KS = 1: four blocks, a wave each,
-// from 8192 blocks on. Every total is formed in a fixed order.
+// from 8192 blocks on or where few tiles stream (WIDE_WAVES, WIDE_SHORT). Every total is formed in a fixed order.
 //
 // Measured, us, rows kernels -> these (forward, dQ, dK/dV), float32 causal: 48 heads x 1024 rows x 32
 // dims 756, 912, 1140 -> 52, 66, 98; 8 x 256 x 64 22, 23, 38 -> 12, 15, 19; 64 x 512 x 64 329, 390, 500
@@ -575,9 +575,10 @@ int launch_wide(SdpaPass pass, const SdpaArgs& a) {
 
 template <typename T, int D>
 int launch_wide_split(SdpaPass pass, const SdpaArgs& a) {
-  const int64_t rows = pass == SDPA_BWD_KV ? a.t_k : a.t_q;
+  const int64_t rows = pass == SDPA_BWD_KV ? a.t_k : a.t_q, streamed = pass == SDPA_BWD_KV ? a.t_q : a.t_k;
   const int64_t waves = a.batch * ((rows + WT - 1) / WT);
-  return waves >= WIDE_WAVES ? launch_wide<T, D, 1>(pass, a) : launch_wide<T, D, 4>(pass, a);
+  const bool alone = waves >= WIDE_WAVES || streamed <= WT || (streamed <= 3 * WT && waves >= WIDE_SHORT);
+  return alone ? launch_wide<T, D, 1>(pass, a) : launch_wide<T, D, 4>(pass, a);
 }
 
 // One storage type's instances (its own translation unit, so they compile in parallel).

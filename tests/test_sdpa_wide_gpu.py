@@ -104,6 +104,18 @@ def test_matches_float64(hipdev, case, dtype):
             np.testing.assert_allclose(g, w, rtol=rel, atol=rel * max(1.0, np.abs(w).max()), err_msg=name)
 
 
+# one streamed tile (a wave a block at any number of blocks), two and three (from 2048 blocks), and the calls of
+# few blocks beside them that stay on the rows kernels
+SHORT_CASES = [(700, 96, 96, 32, 32, True, False), (1030, 64, 40, 80, 64, False, True), (140, 32, 100, 128, 128, False, False),
+               (300, 100, 32, 64, 64, False, True), (129, 32, 32, 16, 16, True, False), (40, 32, 32, 128, 96, True, True), (16, 64, 64, 128, 128, True, False)]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("case", SHORT_CASES, ids=str)
+def test_short_streams_match_float64(hipdev, case, dtype):
+    test_matches_float64(hipdev, case, dtype)
+
+
 def test_hidden_keys_keep_their_garbage_to_themselves(hipdev):
     """Masked keys may hold NaN or infinities: no live row or key sees them."""
     B, t, d = 8, 150, 64
