@@ -307,7 +307,7 @@ class HipDevice(CompiledDevice):
             slots[prog.positions + i] = out.ptr
         for i, p in prog.out_positions:
             bufs[p] = outs[i]
-        check_limn(prog.run(self.lib, slots, self.finish, self.replay_graphs and len(prog.steps) > replay.SHORT_LIST))
+        check_limn(prog.run(self.lib, slots, self.finish, self.replay_graphs and prog.launches > replay.SHORT_LIST))
         for p, i in prog.assigns:
             self.commit(sources[p], outs[i])
             bufs[p] = outs[i]

@@ -12,7 +12,7 @@ one of the outputs the run allocated, in call order. A replay takes its outputs 
 the same few bindings recur run after run), binds every
 slot to this run's buffer and issues the whole list in one call: as a HIP graph captured for that
 binding (one capture serves every later run with the same buffers, and the launches cost the host
-one call), or launch by launch, as a list of at most SHORT_LIST steps always is.
+one call), or launch by launch, as a list of at most SHORT_LIST launches always is.
 
 A recording is refused (the plan keeps running call by call) when two slots share bytes, since a
 pointer into them could not be told apart.
@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import bisect
 import ctypes
+import functools
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -82,6 +83,21 @@ class Program:
     def nslots(self) -> int:
         return self.positions + len(self.out_nbytes)
 
+    @functools.cached_property
+    def launches(self) -> int:
+        """Kernel launches of the list, at most: a contraction given a workspace may fold k slices, one of
+        half widths copy its operands as well; a paired attention backward is two."""
+        total = 0
+        for kind, first in zip(self.steps["kind"].tolist(), self.steps["first"].tolist()):
+            value = lambda k: int(self.args["value"][first + k])
+            if kind in (STEP_MATMUL, STEP_MATMUL_ADD):
+                total += 1 + (value(19 if kind == STEP_MATMUL else 26) > 0)
+            elif kind == STEP_CONTRACT:
+                total += 1 + (value(26) > 0) * (1 if value(3) == 1 else 2)
+            else:
+                total += 2 if kind == STEP_SDPA_BWD else 1
+        return total
+
     def launch(self, lib, slots: np.ndarray, stream=None) -> int:
         return lib.limn_hip_replay(self.steps.ctypes.data, len(self.steps), self.args.ctypes.data, len(self.args),
                                    slots.ctypes.data, len(slots), stream)
@@ -126,10 +142,14 @@ class Program:
         self.graphs.clear()
 
 
-# Lists this short are launched step by step also where graphs are on: a graph launch costs the host
-# some 25 us before its first kernel starts, while of a few launches the first starts at once and the
-# rest are issued under it. A new binding then needs no capture, and nothing is kept for one.
-SHORT_LIST = 6
+# Lists of at most this many kernel launches are issued step by step also where graphs are on: a graph
+# launch costs the host some 20 us before its first kernel starts, while of a few launches the first starts
+# at once and the rest are issued under it; from the eighth on the barrier behind them costs 15 us more. A
+# captured call, us, graph / steps: sums of 2-3 us each, 2 launches 39/23, 5 42/32, 7 44/37, 8 45/52, 9 51/67; of 8
+# us (a split contraction, two launches a step) 6 launches 54/46, 8 61/70; softmax chains 5 50/36, 7 55/47, 9 64/72;
+# attention forward and backward (5) 81/73; 86 steps 2045/2062. A new binding then needs no capture, and
+# nothing is kept for one.
+SHORT_LIST = 7
 GRAPHS_PER_PLAN = 8
 PLANS_KEPT = 64  # launch lists a device keeps, the least recently run dropped first
 ARENAS_PER_PLAN = 3  # a list keeps this many output arenas; past that a replay takes a passing one

@@ -179,3 +179,24 @@ def test_a_short_list_that_fails_is_not_run_again():
     with pytest.raises(RuntimeError):
         dev._replay(plan, prog, {0: dev._alloc(16)})
     assert (lib.graph_calls, lib.list_calls, prog.graph_failure) == (0, 1, None)
+
+
+def test_launches_count_what_a_step_issues():
+    """Split and copying contractions are two and three launches: four split ones are no short list."""
+    def contraction(kind, dtype, ws):
+        n, at = (20, 19) if kind == replay.STEP_MATMUL else (27, 26)
+        args = [0] * n
+        args[3], args[at] = dtype, ws
+        return replay.Launch(kind, tuple(args))
+
+    cases = [(contraction(replay.STEP_MATMUL, 3, 0), 1), (contraction(replay.STEP_MATMUL, 3, 4096), 2), (contraction(replay.STEP_MATMUL_ADD, 2, 4096), 2),
+             (contraction(replay.STEP_CONTRACT, 1, 0), 1), (contraction(replay.STEP_CONTRACT, 1, 64), 2), (contraction(replay.STEP_CONTRACT, 3, 64), 3),
+             (replay.Launch(replay.STEP_ZERO, (0x1000, 16)), 1), (replay.Launch(replay.STEP_SDPA_BWD, (0,) * 20), 2), (replay.Launch(replay.STEP_KERNEL, (1, 2)), 1)]
+    steps, args = replay.bind([c for c, _ in cases], [])
+    assert replay.Program(steps, args, (), (), (), 0).launches == sum(n for _, n in cases)
+    for launch, n in cases:
+        steps, args = replay.bind([launch] * 4, [])
+        lib, prog = StubLib(graph_status=0), replay.Program(steps, args, (), (), (), 1)
+        dev, plan = replaying(lib)
+        dev._replay(plan, prog, {0: dev._alloc(16)})
+        assert (lib.graph_calls, lib.list_calls) == ((1, 0) if 4 * n > replay.SHORT_LIST else (0, 1))
