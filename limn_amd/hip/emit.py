@@ -496,7 +496,11 @@ def contraction_supported(con: Contraction) -> bool:
     if takes_matmul(con):
         return True
     lib, sizes = runtime.kernels(), contract_sizes(con)
-    return bool(lib.limn_hip_contract_pays(*sizes[:5]) and lib.limn_hip_contract_supported(*sizes))
+    return bool(lib.limn_hip_contract_pays(*sizes[:5]) and lib.limn_hip_contract_supported(*sizes)
+                and lib.limn_hip_contract_workspace(*sizes) <= WORKSPACE_CAP)
+
+
+WORKSPACE_CAP = 8 << 30  # the most bytes of copies and partials a contraction may hold beside its operands
 
 
 def contract_us(con: Contraction) -> float:
@@ -2714,6 +2718,7 @@ def nest_runners(dev, nests: list[LoopNest]):
     plans, pairs, inlined, merged = prog.plans, prog.pairs, prog.inlined, prog.merged
     functions = runtime.load_functions(prog.source, prog.names) if prog.names else {}
     runners = []
+    workspace = Workspace(dev)
     operands: dict[int, list] = {}  # a fused contraction's inputs, from its call to its relu's
     producer_inputs: dict[int, list] = {}  # an inlined producer's inputs, from its call to its readers'
     deferred: dict[int, tuple] = {}  # a merged run member's (inputs, outs), from its call to the run's launch
@@ -2740,13 +2745,13 @@ def nest_runners(dev, nests: list[LoopNest]):
             runners.append(_defer_runner(deferred, k))
         elif role == "epilogue" and k in prog.folds:
             source = next(i for i, j in pairs.items() if j == k)
-            runners.append(_fold_runner(dev, prog.folds[k], operands, source))
+            runners.append(_fold_runner(dev, prog.folds[k], operands, source, workspace))
         elif role == "epilogue":
             source = next(i for i, j in pairs.items() if j == k)
-            runners.append(_epilogue_runner(dev, plans[source].contraction, operands, source, prog.addends.get(k),
+            runners.append(_epilogue_runner(dev, plans[source].contraction, operands, source, workspace, prog.addends.get(k),
                                             producer_inputs))
         elif role == "contraction":
-            runners.append(_contraction_runner(dev, plan.contraction))
+            runners.append(_contraction_runner(dev, plan.contraction, workspace))
         else:
             extras = inlined.extras(nest)
             nin = len(nest.kernel.inputs) + len(extras)
@@ -2824,7 +2829,27 @@ def _keep_runner(producer_inputs: dict, k: int):
     return run
 
 
-def _matmul_launcher(dev, con: Contraction, epilogue: int, adds: bool = False):
+class Workspace:
+    """The one workspace of a plan's contractions: split-k partials and the aligned copies of unaligned
+    half-width operands, as large as the largest of them needs. Their launches are ordered on one
+    stream and none keeps anything in it. Allocated on first use and kept with the plan's runners, so a
+    recorded list sees the same pointer every time. Without sharing, an odd-width layer's three products
+    each kept copies of both operands for as long as the plan lived."""
+
+    def __init__(self, dev):
+        self.dev, self.nbytes, self.buf = dev, 0, None
+
+    def reserve(self, nbytes: int) -> None:
+        self.nbytes = max(self.nbytes, nbytes)
+
+    @property
+    def ptr(self) -> int:
+        if self.buf is None:
+            self.buf = self.dev._alloc(self.nbytes)
+        return self.buf.ptr
+
+
+def _matmul_launcher(dev, con: Contraction, epilogue: int, workspace: Workspace, adds: bool = False):
     """launch(inputs, out_ptr, bias_ptr, residual_ptr): the contraction through limn_hip_matmul, or
     through limn_hip_matmul_add when `adds` (the residual read at the output's strides); one that
     neither takes through limn_hip_contract either way."""
@@ -2838,14 +2863,12 @@ def _matmul_launcher(dev, con: Contraction, epilogue: int, adds: bool = False):
     entry, step = (lib.limn_hip_contract, replay.STEP_CONTRACT) if general else (lib.limn_hip_matmul_add, replay.STEP_MATMUL_ADD)
     ws_bytes = int(lib.limn_hip_contract_workspace(*contract_sizes(con)) if general
                    else lib.limn_hip_matmul_workspace(code, con.batch, con.M, con.N, con.K))
-    held: list = []  # the split-k workspace, allocated on first use and kept with the runner
+    workspace.reserve(ws_bytes)
 
     def launch(inputs: list, out: int, bias: int | None = None, res: int | None = None, bias_code: int = code) -> None:
-        if ws_bytes and not held:
-            held.append(dev._alloc(ws_bytes))
         a = inputs[con.a_input].ptr + con.a_offset * size
         b = inputs[con.b_input].ptr + con.b_offset * size
-        ws = held[0].ptr if held else None
+        ws = workspace.ptr if ws_bytes else None
         if adds or general:
             args = (a, b, out, *shape, bias, bias_code, 1, res, con.c_batch, con.c_m, con.c_n, ws, ws_bytes)
             runtime.check_limn(entry(*args, None))
@@ -2859,8 +2882,8 @@ def _matmul_launcher(dev, con: Contraction, epilogue: int, adds: bool = False):
     return launch
 
 
-def _contraction_runner(dev, con: Contraction):
-    launch = _matmul_launcher(dev, con, 0)
+def _contraction_runner(dev, con: Contraction, workspace: Workspace):
+    launch = _matmul_launcher(dev, con, 0, workspace)
 
     def run(inputs: list, outs: list) -> None:
         launch(inputs, outs[0].ptr)
@@ -2879,10 +2902,10 @@ def _stash_runner(operands: dict, k: int):
     return run
 
 
-def _fold_runner(dev, folded: Contraction, operands: dict, k: int):
+def _fold_runner(dev, folded: Contraction, operands: dict, k: int, workspace: Workspace):
     """The batch-sum reader's call: the batched contraction of nest k with its batch folded into
     k, stored into this nest's output (see batch_sum_fold)."""
-    launch = _matmul_launcher(dev, folded, 0)
+    launch = _matmul_launcher(dev, folded, 0, workspace)
 
     def run(inputs: list, outs: list) -> None:
         launch(operands.pop(k), outs[0].ptr)
@@ -2891,7 +2914,7 @@ def _fold_runner(dev, folded: Contraction, operands: dict, k: int):
     return run
 
 
-def _epilogue_runner(dev, con: Contraction, operands: dict, k: int, terms: tuple | None = None,
+def _epilogue_runner(dev, con: Contraction, operands: dict, k: int, workspace: Workspace, terms: tuple | None = None,
                      producer_inputs: dict | None = None):
     """The epilogue reader's call: the contraction of nest k, stored into this nest's output with
     a relu, or (`terms` = (bias input, residual input or None, bias cast nest or None) of this
@@ -2899,13 +2922,13 @@ def _epilogue_runner(dev, con: Contraction, operands: dict, k: int, terms: tuple
     nest's float32 input. Its layout is the contraction's: the reader reads and writes cell for
     cell."""
     if terms is None:
-        launch = _matmul_launcher(dev, con, 1)
+        launch = _matmul_launcher(dev, con, 1, workspace)
 
         def run(inputs: list, outs: list) -> None:
             launch(operands.pop(k), outs[0].ptr)
 
         return run
-    launch = _matmul_launcher(dev, con, 0, adds=True)
+    launch = _matmul_launcher(dev, con, 0, workspace, adds=True)
     bias, res, cast = terms
     from limn_amd.dtypes import ABI_CODE
 

@@ -99,3 +99,52 @@ def test_a_declined_sum_keeps_its_epilogue_nests():
     nests, kept = lowered([(x.transpose() @ w).relu()])
     prog = emit.plan_program(nests, kept, set())
     assert not prog.pairs and all(p.contraction is None for p in prog.plans)
+
+
+class Lib:
+    """liblimn_hip.so's queries; its contraction entry records its arguments instead of running."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        return getattr(emit.runtime.kernels(), name)
+
+    def limn_hip_contract(self, *args):
+        self.calls.append(args)
+        return 0
+
+
+def test_a_plans_contractions_share_one_workspace():
+    """An odd-width layer and its gradients: every product copies operands, and all copies take turns in
+    one allocation of the largest's size."""
+    class Buf:
+        ptr = 0x1000
+
+    class Dev:
+        plan_kept = plan_custom_inputs = tape = None
+
+        def __init__(self):
+            self.lib, self.sizes = Lib(), []
+
+        def _alloc(self, nbytes):
+            self.sizes.append(nbytes)
+            return Buf()
+
+    x, w, dy = (Tensor.from_node(Node(Op.BUFFER, (), bfloat16, s, None)) for s in ((2051, 515), (515, 517), (2051, 517)))
+    nests, _ = lowered([x @ w, dy @ w.transpose(), x.transpose() @ dy])
+    dev = Dev()
+    runners = emit.nest_runners(dev, nests)
+    assert len(runners) == 3
+    for run, nest in zip(runners, nests):
+        run([Buf()] * len(nest.kernel.inputs), [Buf()])
+    needs = [args[-2] for args in dev.lib.calls]
+    assert len(needs) == 3 and min(needs) > 0 and dev.sizes == [max(needs)]
+
+
+def test_a_contraction_of_huge_copies_stays_general():
+    """Copies past WORKSPACE_CAP: a bf16 product whose operands are 16 GB of odd rows each."""
+    a, b = (Tensor.from_node(Node(Op.BUFFER, (), bfloat16, s, None)) for s in ((16, 257, 2000001), (16, 2000001, 255)))
+    nests, kept = lowered([a @ b])
+    (plan,) = [p for n, p in zip(nests, emit.plan_program(nests, kept, set()).plans) if n.kernel.ast.op is Op.SUM]
+    assert plan.contraction is None
