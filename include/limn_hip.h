@@ -177,8 +177,9 @@ int limn_hip_matmul_supported(int dtype, int64_t M, int64_t N, int64_t K, int64_
  * float32 operands, products, totals, result, bias and residual), and bf16 / f16 with operand rows
  * that are not 16-byte aligned or a k that is no multiple of 8 (copied to aligned rows in the
  * workspace first). One stride of each operand must be 1, the other any. Replaces the same reference
- * kernel as limn_hip_matmul (limn/cuda_emit.py:376-685). The workspace rules are limn_hip_matmul's for
- * float32; a half width needs its limn_hip_contract_workspace(...) bytes.
+ * kernel as limn_hip_matmul (limn/cuda_emit.py:376-685). A float32 workspace is optional, as
+ * limn_hip_matmul's is, and 4-byte aligned; a half width needs its
+ * limn_hip_contract_workspace(...) bytes, where that is not 0, 16-byte aligned.
  */
 int limn_hip_contract(const void* a, const void* b, void* c, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                       int64_t a_batch, int64_t a_m, int64_t a_k, int64_t b_batch, int64_t b_k, int64_t b_n, int64_t c_batch,
@@ -202,10 +203,9 @@ int limn_hip_contract_pays(int dtype, int64_t batch, int64_t M, int64_t N, int64
  * buffers. Each step is one launch: a hipRTC module kernel (`function`, `grid` x `block`
  * threads, its arguments the kernel's parameters in order), a zero fill (pointer, bytes), or one
  * call of limn_hip_matmul (its 20 arguments before `stream`), limn_hip_matmul_add or
- * limn_hip_contract (27),
- * limn_hip_sdpa_fwd (13 before
- * `scale`), limn_hip_sdpa_bwd_q (15), limn_hip_sdpa_bwd_kv (16) or limn_hip_sdpa_bwd (17 before
- * `scale`, then passes, workspace and its size: 20), with `scale` in the step. An
+ * limn_hip_contract (27), limn_hip_sdpa_fwd (13 before `scale`), limn_hip_sdpa_bwd_q (15),
+ * limn_hip_sdpa_bwd_kv (16) or limn_hip_sdpa_bwd (17 before `scale`, then passes, workspace and
+ * its size: 20), with `scale` in the step. An
  * argument is `value` when `slot` < 0, else slots[slot] + value: a byte offset into the buffer
  * this replay binds to that slot. Steps run in order on `stream`; the first failing one stops the
  * list and its status is returned. No counterpart in the reference: its capture replays a plan

@@ -273,12 +273,16 @@ int limn_hip_contract(const void* a, const void* b, void* c, int dtype, int64_t 
   MatmulAddends add = {bias, bias_f32, bias_n, residual, r_batch, r_m, r_n, 0};
   if (!half) {
     if (!f32_layout_ok(s)) return fail(LIMN_HIP_EUNSUPPORTED, "contract: operands must be contiguous along m/n or k, within 2 GiB a batch entry");
+    const int64_t used = f32_workspace_bytes(s);
+    if (used > 0 && workspace != nullptr && workspace_bytes >= used && (uintptr_t)workspace % 4 != 0)
+      return fail(LIMN_HIP_EINVAL, "contract: the workspace must be aligned to 4 bytes");
     return launch_matmul_f32(a, b, c, s, epilogue, add, workspace, workspace_bytes, (hipStream_t)stream);
   }
   const bool a_shifted = (uintptr_t)a % 16 != 0, b_shifted = (uintptr_t)b % 16 != 0;
   if (!pack_layout_ok(s, a_shifted, b_shifted))
     return fail(LIMN_HIP_EUNSUPPORTED, "contract: operands must be contiguous along m/n or k, within 2 GiB a batch entry");
-  if (workspace == nullptr || (uintptr_t)workspace % 16 != 0 || workspace_bytes < pack_workspace_bytes(s, a_shifted, b_shifted))
+  const int64_t need = pack_workspace_bytes(s, a_shifted, b_shifted);
+  if (need > 0 && (workspace == nullptr || (uintptr_t)workspace % 16 != 0 || workspace_bytes < need))
     return fail(LIMN_HIP_EINVAL, "contract: a half-width contraction needs its workspace, 16-byte aligned");
   if (bias != nullptr && bias_n == 1 && (uintptr_t)bias % 16 == 0) add.vec |= 1;
   if (residual != nullptr && r_n == 1 && r_m % 8 == 0 && r_batch % 8 == 0 && (uintptr_t)residual % 16 == 0) add.vec |= 2;

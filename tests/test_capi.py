@@ -90,6 +90,24 @@ def test_null_buffers_are_refused():
     assert rc == 1 and "null" in lib.limn_hip_last_error().decode()
 
 
+def test_contract_checks_the_workspace_it_uses():
+    """A split float32 contraction writes partial tiles to its workspace, so its alignment is checked
+    (0x1002 is none); a half width is refused without the copies' bytes."""
+    lib = runtime.kernels()
+    sizes = (1, 64, 64, 4096, 0, 4096, 1, 0, 64, 1)
+
+    def call(dtype, a, sizes, ws, room):
+        return lib.limn_hip_contract(a, FAKE, FAKE, dtype, *sizes, 0, 64, 1, 0, None, dtype, 1, None, 0, 0, 0, ws, room, None)
+
+    need = lib.limn_hip_contract_workspace(1, *sizes, 0)
+    assert need > 0
+    assert call(1, FAKE, sizes, ctypes.c_void_p(0x1002), need) == 1 and "aligned to 4" in lib.limn_hip_last_error().decode()
+    odd = (1, 64, 64, 4097, 0, 4097, 1, 0, 64, 1)
+    need = lib.limn_hip_contract_workspace(3, *odd, 0)
+    assert call(3, FAKE, odd, ctypes.c_void_p(0x1008), need) == call(3, FAKE, odd, FAKE, need - 1) == call(3, FAKE, odd, None, 0) == 1
+    assert "16-byte" in lib.limn_hip_last_error().decode()
+
+
 def test_every_split_fits_the_static_scratch():
     """limn_hip_matmul_noalloc keeps split-k slices in a static array of LIMN_HIP_SCRATCH_BYTES.
     The planner splits only while output tiles x slices stay under two waves of 256 workgroups,
