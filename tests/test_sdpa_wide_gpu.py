@@ -307,6 +307,26 @@ def test_split_probabilities_of_far_scores(hipdev, hd, hv, dtype, size):
     np.testing.assert_allclose(lse[clear], s[..., -1][clear], rtol=(hd + 2) * 2.0**-23)
 
 
+@pytest.mark.parametrize("hd", [32, 80, 120])
+def test_a_score_past_float32_stays_in_its_row(hipdev, hd):
+    """Finite bfloat16 queries and keys whose score is infinite: NaN in that row, as exp(inf - inf) is, a
+    weight of 0 where it is -inf, and every other row of the workgroup's second walk as without it."""
+    B, tq, tk = 16, 40, 130
+    rng = np.random.default_rng(hd)
+    q, k, v = (rng.standard_normal(s) for s in ((B, tq, hd), (B, tk, hd), (B, tk, hd)))
+    q[:, 5], q[:, 6], k[:, 70] = 1e20, -1e20, 1e20
+    out, lse = forward(hipdev, "bfloat16", q, k, v, hd**-0.5)
+    assert np.isnan(out[:, 5]).all() and np.isnan(lse[:, 5]).all()
+    q, k, v = (stored(x, "bfloat16")[1] for x in (q, k, v))
+    top = np.argmax(q @ k.swapaxes(1, 2), axis=-1)
+    rest = np.delete(np.arange(tq), 5)
+    sure = np.abs(q.sum(-1)) > 1  # rows whose score with key 70 is far from the others, whatever its rounding
+    want = np.take_along_axis(v, top[..., None], 1)
+    assert np.isfinite(out[:, rest]).all() and sure.mean() > 0.7
+    np.testing.assert_array_equal(out[:, rest][(sure & (top == 70))[:, rest]], want[:, rest][(sure & (top == 70))[:, rest]])
+    np.testing.assert_array_equal(out[:, 6], want[:, 6])
+
+
 @pytest.mark.parametrize("hd", [24, 32, 48, 80, 96, 128])
 def test_a_far_score_keeps_its_whole_weight(hipdev, hd):
     """Queries in line with one key, its score thousands above the others': a weight of exactly 1, whatever
