@@ -23,9 +23,9 @@
 // from 8192 blocks on or where few tiles stream (WIDE_WAVES, WIDE_SHORT). Every total is formed in a fixed order.
 //
 // Measured, us, rows kernels -> these (forward, dQ, dK/dV), float32 causal: 48 heads x 1024 rows x 32
-// dims 756, 912, 1140 -> 52, 66, 98; 8 x 256 x 64 22, 23, 38 -> 12, 15, 19; 64 x 512 x 64 329, 390, 500
-// -> 40, 56, 88 (paired blocks; unpaired 57, 71, 100); 16 x 2048 x 64, full, 1252, 1531, 2125 -> 191,
-// 266, 410 (90 TFLOP/s); f16, 256 heads, 197 x 1021 x 80, key mask 3015, 3765, 2552 -> 407, 616, 797.
+// dims 756, 912, 1140 -> 48, 60, 90; 8 x 256 x 64 22, 23, 38 -> 12, 15, 19; 64 x 512 x 64 329, 390, 500
+// -> 40, 56, 88 (paired blocks; unpaired 57, 71, 100); 16 x 2048 x 64, full, 1252, 1531, 2125 -> 178,
+// 246, 421 (90 TFLOP/s); f16, 256 heads, 197 x 1021 x 80, key mask, dQ and dK/dV 3765, 2552 -> 480, 692.
 //
 // Accuracy: a tile's product starts from zero and is added to the running total once per tile (with
 // the forward's rescale, one fused operation), so a total over thousands of rows is a sum of
